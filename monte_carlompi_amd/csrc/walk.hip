@@ -48,14 +48,19 @@ constexpr int CUR_SLOT_SHIFT = 28;
 constexpr uint32_t CUR_OFF_MASK = (1u << CUR_SLOT_SHIFT) - 1u;
 
 // Take the block's chunk number `seq` into free slot `slot` (whole wave calls).
-// Returns false when the global queue is empty.
-template <class BS>
+// Returns false when the global queue is empty.  ONE: the block's only chunk
+// is the one of its own number (k_walk's ONE), no queue.
+template <bool ONE = false, class BS>
 __device__ bool acquire_chunk(BS &bs, uint32_t seq, int slot, const KParams &P)
 {
     const int lane = lane_id();
     unsigned int j = 0;
-    if (lane == 0) j = atomicAdd(P.chunk_counter, 1u);
-    j = (unsigned int)bcast((int)j, 0);
+    if constexpr (ONE) {
+        j = blockIdx.x;
+    } else {
+        if (lane == 0) j = atomicAdd(P.chunk_counter, 1u);
+        j = (unsigned int)bcast((int)j, 0);
+    }
     if (j >= P.n_chunks) {
         if (lane == 0) __atomic_store_n(&bs.exhausted, 1, __ATOMIC_RELAXED);
         return false;
@@ -496,8 +501,13 @@ __device__ __forceinline__ void set_priority(uint32_t i)
 // slots of the block (tally slots in LDS, 5.3 KB each); the polarised walk
 // in blocks of up to 256 threads takes 2, so that with its tables and tail
 // packets three blocks fit in a CU's LDS (with 4, two do; larger blocks keep
-// 4, or their waves would wait for slots held by lingering walks).
-template <class W, int WPE, bool DIRECT = false, int SL = SLOTS>
+// 4, or their waves would wait for slots held by lingering walks).  ONE: one
+// chunk of at most `block` photons per block, dealt to its waves evenly at the
+// start (P.take each) and no refill after: walks whose photons all fit in the
+// launch's lanes (walk_shape).  The waves then enter their tail mode at once
+// or after a short drain, on every SIMD of the chip, instead of a few blocks
+// working through full-size chunks (measured at walk_shape).
+template <class W, int WPE, bool DIRECT = false, int SL = SLOTS, bool ONE = false>
 __global__ void __launch_bounds__(W::MAX_BLOCK) __attribute__((amdgpu_waves_per_eu(WPE)))
 k_walk(const KParams P)
 {
@@ -522,8 +532,11 @@ k_walk(const KParams P)
     __syncthreads();
     if (threadIdx.x == 0) bs.holders = blockDim.x >> 6;
     if (wave == 0) {
-        if (!acquire_chunk(bs, 0u, 0, P)) {
+        if (!acquire_chunk<ONE>(bs, 0u, 0, P)) {
             if (lane == 0) bs.hdr[0].seqcount = 0ull;  // seq 0, count 0
+        }
+        if constexpr (ONE) {
+            if (lane == 0) bs.exhausted = 1;
         }
     }
     __syncthreads();
@@ -535,12 +548,23 @@ k_walk(const KParams P)
     uint64_t my_gid = 0;
     int spins = 0;
     bool to_coop = false;
+    if constexpr (ONE) {
+        // wave k takes photons [k take, (k + 1) take) of the chunk
+        const uint32_t off = (uint32_t)wave * P.take + (uint32_t)lane;
+        const SlotHdr &H = bs.hdr[0];
+        if ((uint32_t)lane < P.take && off < (uint32_t)lds_load(&H.seqcount)) {
+            my_gid = H.gid0 + off;
+            state = w.start(P, H.case_id, H.p0 + off, my_gid) ? DONE : LIVE;
+        }
+    }
 
     for (;;) {
         // ---------------- cold: retire finished lanes, refill empty ones
         if (__ballot(state == DONE)) retire<W, DIRECT>(bs, P, w, state, my_slot, my_gid);
-        const bool exhausted = lds_load(&bs.exhausted) != 0;
-        if (!exhausted && __ballot(state == EMPTY)) refill(bs, P, w, state, my_slot, my_gid);
+        if constexpr (!ONE) {
+            const bool exhausted = lds_load(&bs.exhausted) != 0;
+            if (!exhausted && __ballot(state == EMPTY)) refill(bs, P, w, state, my_slot, my_gid);
+        }
         const unsigned long long live = __ballot(state == LIVE);
         if (live == 0ull) {
             // photons can finish at hand-out (first step, surface mode): retire first
@@ -1427,12 +1451,89 @@ int mcs_get_launch(const mcs_ctx *c, mcs_launch *out)
 
 static int finish_walk(mcs_ctx *c);
 
-// Photons per chunk of a walk: the launch's, raised to the block's threads.
-// A block holds at most its tally slots' worth of chunks, each until its
-// longest walk ends; chunks much smaller than the block left most of its
-// lanes idle while the queue still had work (489-photon chunks in
-// 1024-thread blocks: 6.3 ms for the 1e6-photon case, 0.7 ms at 977).
-static int walk_chunk(const mcs_ctx *c) { return std::max(c->launch.chunk, c->launch.block); }
+// The launch shape of a walk, from the context's and the photon count.
+struct WalkShape {
+    int block, grid;    // threads per block; blocks that fill the launch's share of the chip
+    int chunk;          // photons per chunk
+    int64_t n_chunks;   // over all cases
+    int take;           // > 0: k_walk's ONE form, this many photons per wave
+};
+
+static int64_t count_chunks(const mcs_ctx *c, int chunk)
+{
+    int64_t n = 0;
+    for (const DevCase &D : c->dcases) n += (D.n_photons + chunk - 1) / chunk;
+    return n;
+}
+
+// * Chunks are at least the block's threads: a block holds at most its tally
+//   slots' worth of chunks, each until its longest walk ends; chunks much
+//   smaller than the block left most of its lanes idle while the queue still
+//   had work (489-photon chunks in 1024-thread blocks: 6.3 ms for the
+//   1e6-photon case, 0.7 ms at 977).
+// * With fewer photons than one such chunk per block, blocks would stay
+//   without work (10,000 photons in 2048-photon chunks: 5 blocks).  Walks whose
+//   records do not depend on the shape (coop_live 0, polarised, replay) then
+//   shrink their chunks to one per block (500,000 photons at the default
+//   shape, coop_live 0: kernel 2.00 -> 1.86 ms; polarised 300,000: 1.89 -> 1.32).
+// * Native walks that have a lane for every photon take the ONE form of k_walk:
+//   as many blocks as are resident together, the photons spread evenly over
+//   them.  Kernel ms at the default shape (256, 4, 2048, 8), queue -> ONE:
+//   coop_live 0: 2,000 photons 1.50 -> 0.70, 10,000 1.53 -> 0.76, 250,000 1.98
+//   -> 1.54; polarised: 2,000 1.51 -> 0.43, 20,000 1.82 -> 0.77, 100,000 1.96 ->
+//   1.02.  Polarised blocks of 512 threads, one per CU, hold the photons up to
+//   8 waves per CU (20,000 photons: 0.77 ms; 256-thread blocks, three per CU,
+//   0.95: three waves share a SIMD from the start, and not evenly), then
+//   256-thread blocks up to 12.  In the cooperative mode the form is taken when
+//   its waves hold at most coop_live photons each, so that they start in the
+//   tail (10,000 photons 0.90 -> 0.08 ms, 50,000 0.94 -> 0.12); above that the
+//   caller's shape says how many photons finish cooperatively.
+static WalkShape walk_shape(const mcs_ctx *c, int mode)
+{
+    WalkShape s;
+    const bool replay = mode == MCS_REPLAY, polar = !replay && c->polar;
+    const int coop = c->launch.coop_live;
+    const int64_t n = c->total_photons;
+    s.block = replay ? std::min(c->launch.block, ReplayWalker::MAX_BLOCK) : c->launch.block;
+    int per_cu = c->launch.blocks_per_cu;
+    if (polar && s.block > PolarWalker::MAX_BLOCK) {
+        per_cu *= s.block / PolarWalker::MAX_BLOCK;   // same threads per CU in smaller blocks
+        s.block = PolarWalker::MAX_BLOCK;
+    }
+    if (!replay && n > 0) {
+        int block = s.block, blocks = std::min(per_cu, 16 / (s.block / 64));
+        if (polar) {
+            const bool eight = n <= (int64_t)512 * c->cus;
+            block = eight ? 512 : 256;
+            blocks = eight ? 1 : 3;
+        }
+        const int64_t g = (int64_t)std::max(blocks, 1) * c->cus;
+        const int64_t ch = (n + g - 1) / g;
+        const int waves = block / 64;
+        const int64_t take = (ch + waves - 1) / waves;
+        if (ch <= block && (polar || coop == 0 || take <= coop)) {
+            const int64_t nch = count_chunks(c, (int)ch);
+            if (nch <= g) {
+                s.block = block;
+                s.grid = (int)nch;
+                s.chunk = (int)ch;
+                s.n_chunks = nch;
+                s.take = (int)take;
+                return s;
+            }
+        }
+    }
+    s.take = 0;
+    s.grid = per_cu * c->cus;
+    s.chunk = std::max(c->launch.chunk, c->launch.block);
+    if (replay || polar || coop == 0) {
+        const int64_t per_block = (n + s.grid - 1) / s.grid;
+        s.chunk = (int)std::min<int64_t>(s.chunk, std::max<int64_t>(per_block, c->launch.block));
+    }
+    s.n_chunks = count_chunks(c, s.chunk);
+    if (s.grid > s.n_chunks) s.grid = (int)std::max<int64_t>(s.n_chunks, 1);
+    return s;
+}
 
 static uint64_t mix64(uint64_t h, uint64_t v)
 {
@@ -1441,23 +1542,17 @@ static uint64_t mix64(uint64_t h, uint64_t v)
 }
 
 // enqueue fill + walk + scatter on the context stream
-static int enqueue_walk(mcs_ctx *c, int mode, const KParams &P, uint32_t n_chunks, int64_t n, bool records,
+static int enqueue_walk(mcs_ctx *c, int mode, const KParams &P, const WalkShape &shape, int64_t n, bool records,
                         bool events)
 {
+    const uint32_t n_chunks = (uint32_t)shape.n_chunks;
+    const int block = shape.block, grid = shape.grid;
     const int nc = (int)c->cases.size();
     const uint64_t nclear = (uint64_t)(TF + TU) * nc + 16;
     const unsigned blocks_clear = (unsigned)std::min<uint64_t>((nclear + 255) / 256, 1024);
     hipLaunchKernelGGL(k_clear, dim3(blocks_clear), dim3(256), 0, c->stream,
                        (unsigned long long *)P.tally_f, (uint64_t)TF * nc, P.tally_u, (uint64_t)TU * nc,
                        P.ctl, (uint64_t)16);
-    int block = (mode == MCS_REPLAY) ? std::min(c->launch.block, ReplayWalker::MAX_BLOCK)
-                                     : c->launch.block;
-    int grid = c->launch.blocks_per_cu * c->cus;
-    if (mode == MCS_NATIVE && c->polar && block > PolarWalker::MAX_BLOCK) {
-        grid *= block / PolarWalker::MAX_BLOCK;   // same threads per CU in smaller blocks
-        block = PolarWalker::MAX_BLOCK;
-    }
-    if ((uint32_t)grid > n_chunks) grid = (int)std::max<uint32_t>(n_chunks, 1u);
     // events bracket the walk kernel alone: kernel_ms is its device time
     if (events && hipEventRecord(c->ev0, c->stream) != hipSuccess)
         return set_err(c, MCS_ERR_HIP, "hipEventRecord failed");
@@ -1467,8 +1562,12 @@ static int enqueue_walk(mcs_ctx *c, int mode, const KParams &P, uint32_t n_chunk
         // + the tail mode's owner lanes and packets (16 ints and PK_SLOTS packets a wave)
         const size_t lds = (size_t)P.pm_lds_floats * sizeof(float) +
                            (size_t)(block / 64) * (16 * sizeof(int) + PK_SLOTS * sizeof(PolarPacket)) + 16;
-        // blocks of up to 256 threads: two chunk slots (k_walk's SL)
-        if (P.rec_direct) {
+        // blocks of up to 256 threads: two chunk slots (k_walk's SL); ONE holds one
+        if (shape.take > 0 && P.rec_direct) {
+            hipLaunchKernelGGL((k_walk<PolarWalker, 3, true, 1, true>), dim3(grid), dim3(block), lds, c->stream, P);
+        } else if (shape.take > 0) {
+            hipLaunchKernelGGL((k_walk<PolarWalker, 3, false, 1, true>), dim3(grid), dim3(block), lds, c->stream, P);
+        } else if (P.rec_direct) {
             if (block <= 256)
                 hipLaunchKernelGGL((k_walk<PolarWalker, 3, true, 2>), dim3(grid), dim3(block), lds, c->stream, P);
             else
@@ -1483,7 +1582,8 @@ static int enqueue_walk(mcs_ctx *c, int mode, const KParams &P, uint32_t n_chunk
         // the instance whose register budget fits the shape's waves per SIMD:
         // <= 4 (1024-thread blocks, one per CU) 128 VGPRs, 5 96, more 80 (the
         // 6-wave build's spills sit outside the step loop)
-        const int waves_per_simd = (c->launch.blocks_per_cu * (block / 64) + 3) / 4;
+        // (ONE is built for 4 and keeps at most that many resident)
+        const int waves_per_simd = shape.take > 0 ? 4 : (c->launch.blocks_per_cu * (block / 64) + 3) / 4;
         // cooperative tables, or at coop_live 0 the packet tail's owners and
         // packets (in the build that carries it)
         const size_t tab = c->launch.coop_live > 0
@@ -1491,7 +1591,11 @@ static int enqueue_walk(mcs_ctx *c, int mode, const KParams &P, uint32_t n_chunk
                            : waves_per_simd <= 4
                                ? (size_t)(block / 64) * (HG_TAIL * sizeof(int) + HG_PK_SLOTS * sizeof(HgPacket))
                                : 0;
-        if (waves_per_simd > 5 && P.rec_direct)
+        if (shape.take > 0 && P.rec_direct)
+            hipLaunchKernelGGL((k_walk<NativeWalker, 4, true, SLOTS, true>), dim3(grid), dim3(block), tab, c->stream, P);
+        else if (shape.take > 0)
+            hipLaunchKernelGGL((k_walk<NativeWalker, 4, false, SLOTS, true>), dim3(grid), dim3(block), tab, c->stream, P);
+        else if (waves_per_simd > 5 && P.rec_direct)
             hipLaunchKernelGGL((k_walk<NativeWalker, 6, true>), dim3(grid), dim3(block), tab, c->stream, P);
         else if (waves_per_simd > 5)
             hipLaunchKernelGGL((k_walk<NativeWalker, 6>), dim3(grid), dim3(block), tab, c->stream, P);
@@ -1588,7 +1692,8 @@ int mcs_walk(mcs_ctx *c, const mcs_walk_args *a)
         rlen = a->replay_off[n];
     }
     // chunking
-    const int chunk = walk_chunk(c);
+    const WalkShape shape = walk_shape(c, a->mode);
+    const int chunk = shape.chunk;
     std::vector<int32_t> chunk0(nc + 1);
     int64_t nch = 0;
     for (int k = 0; k < nc; ++k) {
@@ -1632,6 +1737,7 @@ int mcs_walk(mcs_ctx *c, const mcs_walk_args *a)
     P.case_chunk0 = (const int32_t *)c->d_chunk0.p;
     P.n_cases = nc;
     P.chunk = chunk;
+    P.take = (uint32_t)shape.take;
     P.n_chunks = (uint32_t)nch;
     P.refill_min = (uint32_t)c->launch.refill_min;
     P.coop_live = c->launch.coop_live;
@@ -1676,7 +1782,7 @@ int mcs_walk(mcs_ctx *c, const mcs_walk_args *a)
             if (c->gexec) { (void)hipGraphExecDestroy(c->gexec); c->gexec = nullptr; }
             if (c->graph) { (void)hipGraphDestroy(c->graph); c->graph = nullptr; }
             HIPCHK(c, hipStreamBeginCapture(c->stream, hipStreamCaptureModeThreadLocal));
-            int er = enqueue_walk(c, a->mode, P, (uint32_t)nch, n, records, false);
+            int er = enqueue_walk(c, a->mode, P, shape, n, records, false);
             hipGraph_t g = nullptr;
             hipError_t ee = hipStreamEndCapture(c->stream, &g);
             if (er) { if (g) (void)hipGraphDestroy(g); return er; }
@@ -1690,7 +1796,7 @@ int mcs_walk(mcs_ctx *c, const mcs_walk_args *a)
         HIPCHK(c, hipGraphLaunch(c->gexec, c->stream));
         HIPCHK(c, hipEventRecord(c->ev1, c->stream));
     } else {
-        if ((r = enqueue_walk(c, a->mode, P, (uint32_t)nch, n, records, true))) return r;
+        if ((r = enqueue_walk(c, a->mode, P, shape, n, records, true))) return r;
     }
     c->last_mode = a->mode;
     c->last_records = records;
@@ -1729,9 +1835,9 @@ int mcs_walk_noalloc(mcs_ctx *c, const mcs_walk_args *a, const mcs_dev_out *o)
         int r = finish_walk(c);
         if (r) return r;
     }
-    const int chunk = walk_chunk(c);
-    int64_t nch = 0;
-    for (int k = 0; k < nc; ++k) nch += (c->dcases[k].n_photons + chunk - 1) / chunk;
+    const WalkShape shape = walk_shape(c, MCS_NATIVE);
+    const int chunk = shape.chunk;
+    const int64_t nch = shape.n_chunks;
     if (nch > 0x7FFFFFFF) return set_err(c, MCS_ERR_ARG, "too many chunks; raise the chunk size");
     c->last_records = c->last_stokes = false;
     unsigned long long *const scr = c->noalloc_scratch;   // this device's scratch
@@ -1743,6 +1849,7 @@ int mcs_walk_noalloc(mcs_ctx *c, const mcs_walk_args *a, const mcs_dev_out *o)
     P.case_chunk0 = chunk0;
     P.n_cases = nc;
     P.chunk = chunk;
+    P.take = (uint32_t)shape.take;
     P.n_chunks = (uint32_t)nch;
     P.refill_min = (uint32_t)c->launch.refill_min;
     P.coop_live = c->launch.coop_live;
@@ -1770,7 +1877,7 @@ int mcs_walk_noalloc(mcs_ctx *c, const mcs_walk_args *a, const mcs_dev_out *o)
     }
     c->h_sum[7] = 0ull;   // set again by this walk's k_summary
     hipLaunchKernelGGL(k_chunk_table, dim3(1), dim3(1024), 0, c->stream, P.cases, nc, chunk, chunk0);
-    int r = enqueue_walk(c, MCS_NATIVE, P, (uint32_t)nch, n, false, true);
+    int r = enqueue_walk(c, MCS_NATIVE, P, shape, n, false, true);
     if (r) return r;
     c->last_mode = MCS_NATIVE;
     c->last_tallies_ctx = false;
