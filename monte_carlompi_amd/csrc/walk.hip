@@ -389,97 +389,142 @@ __device__ __forceinline__ bool hot_walk_step(W &w, const KParams &P)
 
 // Tail mode of the reproducible HG walk (coop_live = 0).  Once the queue is
 // empty and a wave holds at most HG_TAIL photons, the wave works in rounds as
-// the polarised tail does: the G = HG_PK / 2^ceil(log2 L) lanes of group g
+// the polarised tail does: the G = 64 / 2^ceil(log2 L) lanes of group g
 // build the packets of the next G steps of the group's photon (Philox block,
 // free path, cos theta, the azimuth's sine and cosine: hg_packet), then every
-// photon's own lane walks those G steps through hg_move -- rotation, move and
-// event test, ~25 instructions instead of the whole step -- until the step in
-// which any photon of the wave has an event or reaches the step cap, or the
-// last packet (a wave-uniform exit).  The packet and the move use the
-// expressions of NativeWalkerT::step and the event its hg_event, so records
+// photon's own lane walks those G steps.  What ends a launch is the longest
+// walk's serial chain there, so a step of it is kept to the rotation and the
+// move: HG_BATCH steps run straight, with one test for any exit or
+// near-vertical direction among them; a batch with one (rare) is dropped
+// and walked again step by step through hg_move, which tests every step.  The
+// vertical direction cosine and the depth do not depend on the horizontal
+// ones, so a batch runs as two chains: hg_dive (five dependent operations a
+// step, the test) and, beside the next batch's, hg_swing.
+// Absorption needs no state: the packets' lanes find each photon's first
+// absorbing step, and the round ends there for the whole wave (a wave-uniform
+// count).  The groups keep their photons' constants while the same photons
+// are live and none had an event.  The packet, hg_dive, hg_swing and hg_move use
+// the expressions of NativeWalkerT::step and the event its hg_event, so records
 // equal the one-lane walk's bit for bit.  LDS (the dynamic area, which holds
-// no cooperative tables at coop_live = 0): HG_TAIL owner lanes and
-// HG_PK_SLOTS packets per wave.
+// no cooperative tables at coop_live = 0): one HgTab per wave.  A lone wave
+// with one photon (100 photons, longest walk 3,035 steps) takes 66 ns a step
+// instead of 170 with an event test per step: ~95 vector instructions a batch,
+// issue-bound; 10,000 photons 0.76 -> 0.41 ms, 1e6 at (1024, 1) 2.23 -> 1.65.
 constexpr int HG_TAIL = 16;
-constexpr int HG_PK_LOG = 6;
-constexpr int HG_PK = 1 << HG_PK_LOG;
-constexpr int HG_PK_SLOTS = HG_PK + 1;   // the last group's prefetch may read one past
-template <int WPE>
-constexpr bool HG_TAIL_IN = WPE <= 4;    // the builds that carry the packet tail
-// live photons at which a wave with the queue dry leaves the hot loop for its
-// tail: the cooperative tail's threshold, or the packet tail's at coop_live 0
-template <int WPE>
-__device__ __forceinline__ int tail_live(const KParams &P)
-{
-    if constexpr (HG_TAIL_IN<WPE>) return P.coop_live > 0 ? P.coop_live : HG_TAIL;
-    else return P.coop_live;
-}
-// (a template, so that only the builds that carry it instantiate it: another
-// caller of the walker's non-inlined helpers changes how the others inline)
-template <int WPE>
+// the last group's prefetches may read two batches past its steps
+constexpr int HG_SLOTS = 64 + 2 * HG_BATCH;
+// A wave's packets in LDS: step k of the photon of rank r at [r G + k].
+struct HgTab {
+    float4 rot[HG_SLOTS];       // cos and sin theta, sin and cos phi
+    float dt[HG_SLOTS];         // free path
+    uint32_t w[HG_SLOTS];       // absorption word
+    int own[HG_TAIL];           // lanes of the live photons, by rank
+};
+static_assert(sizeof(HgTab) % 16 == 0, "HgTab: 16-byte LDS loads");
 __device__ void hg_tail(NativeWalker &w, int &state, const KParams &P, int wave)
 {
     extern __shared__ __align__(16) CoopEntry coop_tab[];
-    int *const owners = reinterpret_cast<int *>(coop_tab);
-    HgPacket *const pk = reinterpret_cast<HgPacket *>(owners + (blockDim.x >> 6) * HG_TAIL) + wave * HG_PK_SLOTS;
-    int *const own = owners + wave * HG_TAIL;
+    HgTab &tab = reinterpret_cast<HgTab *>(coop_tab)[wave];
     const int lane = lane_id();
+    unsigned long long em = 0ull;              // live photons of the grouping (0: regroup)
+    int lg = 0, G = 64;
+    PhiloxPre pre{};
+    uint32_t io = 0u, t_abs = 0u;
+    float ca = 0.f, cb = 0.f, ccc = 0.f, cd = 0.f, ce = 0.f;
+    bool iso = false, member = false;
     for (;;) {
         const unsigned long long live = __ballot(state == LIVE);
         if (live == 0ull) break;
-        const int L = __popcll(live);
-        const int lg = (L <= 1) ? 0 : 32 - __clz(L - 1);
-        const int G = HG_PK >> lg;                 // >= 2 (L <= HG_TAIL)
-        if (state == LIVE) own[lane_rank(live)] = lane;
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
-        const int g = lane >> (HG_PK_LOG - lg);    // >= L for lanes >= HG_PK
-        const int o = own[g < L ? g : 0];
-        const uint32_t ck0 = bperm(o, w.pre.ck0), h0 = bperm(o, w.pre.h0), l0 = bperm(o, w.pre.l0);
-        const uint32_t io = bperm(o, w.i);
-        const float ca = bperm(o, w.a), cb = bperm(o, w.b), ccc = bperm(o, w.cc), cd = bperm(o, w.d), ce = bperm(o, w.e);
-        const bool iso = bperm(o, (uint32_t)w.iso) != 0u;
-        if (g < L) {
-            const PhiloxPre pre{ck0, h0, l0};
+        if (live != em) {
+            em = live;
+            const int L = __popcll(live);
+            lg = (L <= 1) ? 0 : 32 - __clz(L - 1);
+            G = 64 >> lg;                      // >= HG_BATCH (L <= HG_TAIL)
+            if (state == LIVE) tab.own[lane_rank(live)] = lane;
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+            const int g = lane >> (6 - lg);
+            member = g < L;
+            const int o = tab.own[member ? g : 0];
+            pre = PhiloxPre{bperm(o, w.pre.ck0), bperm(o, w.pre.h0), bperm(o, w.pre.l0)};
+            io = bperm(o, w.i);
+            t_abs = bperm(o, w.t_abs_all);
+            ca = bperm(o, w.a); cb = bperm(o, w.b); ccc = bperm(o, w.cc); cd = bperm(o, w.d); ce = bperm(o, w.e);
+            iso = bperm(o, (uint32_t)w.iso) != 0u;
+        }
+        bool absorbed;
+        {
             const u32x4 cur = philox_step(pre, io + 1u + (uint32_t)(lane & (G - 1)), P.key0, P.key1);
             HgPacket q;
             NativeWalker::hg_packet(cur, ca, cb, ccc, cd, ce, iso, q);
-            pk[lane] = q;
+            tab.rot[lane] = make_float4(q.cost, q.sint, q.sinp, q.cosp);
+            tab.dt[lane] = q.dtau;
+            tab.w[lane] = q.w;
+            absorbed = member && q.w < t_abs;
         }
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
+        // steps of this round: up to the first absorption of any photon; one by
+        // one for a wave that holds a photon near the step cap (photons in the
+        // tail have i < max_steps, so the first step is always taken)
+        unsigned long long am = __ballot(absorbed);
+        for (int h = 32; h >= G; h >>= 1) am |= am >> h;
+        am &= G == 64 ? ~0ull : (1ull << G) - 1ull;
+        int ns = am ? __ffsll((long long)am) : G;
+        if (__ballot(state == LIVE && P.max_steps - w.i < (uint32_t)G)) ns = 1;
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        int k = 0;
+        bool done = false;
         if (state == LIVE) {
-            // photons in the tail have i < max_steps: the first step is taken
-            const HgPacket *const mine = pk + lane_rank(live) * G;
-            uint32_t cap = P.max_steps;
-            asm volatile("" : "+v"(cap));
-            HgPacket a = mine[0];
-            int k = 0;
-            for (;;) {
-                const HgPacket b = mine[k + 1];
-                bool ev = w.hg_move(a);
-                ++k;
-                if (__ballot(ev || w.i >= cap) != 0ull || k >= G) break;
-                a = mine[k + 1];
-                ev = w.hg_move(b);
-                ++k;
-                if (__ballot(ev || w.i >= cap) != 0ull || k >= G) break;
+            const int at = lane_rank(live) * G;
+            const float4 *const rot = tab.rot + at;
+            const float *const dt = tab.dt + at;
+            if (ns >= HG_BATCH) {
+                // a batch's depth chain (hg_dive), then its horizontal turns
+                // (hg_swing) beside the next batch's chain
+                const float cap = -w.tau_tot;
+                HgBatch p, q;
+                w.hg_load(p, rot, dt);
+                w.hg_load(q, rot + HG_BATCH, dt + HG_BATCH);
+                float u = w.muz, z = w.z;
+                // `a` went well: count it and swing it beside `b`'s dive; its
+                // registers take the batch after `b`.  Past the round's last
+                // batch the dive and the loads go unused: the asm keeps both
+                // chains in one block, ahead of the branch.
+                const auto next = [&](HgBatch &a, HgBatch &b) {
+                    w.muz = u; w.z = z;
+                    k += HG_BATCH;
+                    w.hg_swing(a);
+                    w.hg_load(a, rot + k + HG_BATCH, dt + k + HG_BATCH);
+                    float e = NativeWalker::hg_dive(b, u, z, cap);
+                    if (k + HG_BATCH > ns) e = 1.f;
+                    asm volatile("" : "+v"(e), "+v"(w.mux), "+v"(w.muy), "+v"(w.tau_acc));
+                    return __ballot(e > 0.f) == 0ull;
+                };
+                if (__ballot(NativeWalker::hg_dive(p, u, z, cap) > 0.f) == 0ull)
+                    while (next(p, q) && next(q, p)) {}
+                w.i += (uint32_t)k;
             }
-            // the last step's event test, formed again from the state it left
-            const HgPacket &last = mine[k - 1];
-            const bool ev = w.z > 0.f || w.z < -w.tau_tot || last.w < w.t_abs_all;
-            bool d = false;
-            if (ev) {
+            while (k < ns) {
+                const float4 r = rot[k];
+                const HgPacket q{dt[k], 0u, r.x, r.y, r.z, r.w};
+                w.hg_move(q);
+                ++k;
+                if (__ballot(w.z > 0.f || w.z < -w.tau_tot) != 0ull) break;
+            }
+            const uint32_t lw = tab.w[at + k - 1];
+            bool ended = false;
+            if (w.z > 0.f || w.z < -w.tau_tot || lw < w.t_abs_all) {
                 w.r = philox_step(w.pre, w.i + 1u, P.key0, P.key1);   // the next step's block (re-emission)
-                d = w.hg_event(P, last.dtau, last.w);
+                ended = w.hg_event(P, dt[k - 1], lw);
+                done = true;
             }
-            if (d || w.i >= P.max_steps) {
-                if (!d) w.cond = 0;
+            if (ended || w.i >= P.max_steps) {
+                if (!ended) w.cond = 0;
                 state = DONE;
             }
         }
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
+        // photons that had an event took steps of their own: regroup
+        if (__ballot(done)) em = 0ull;
+        else io += (uint32_t)__builtin_amdgcn_readlane(k, __ffsll((long long)live) - 1);
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
     }
 }
 
@@ -507,11 +552,14 @@ __device__ __forceinline__ void set_priority(uint32_t i)
 // launch's lanes (walk_shape).  The waves then enter their tail mode at once
 // or after a short drain, on every SIMD of the chip, instead of a few blocks
 // working through full-size chunks (measured at walk_shape).
-template <class W, int WPE, bool DIRECT = false, int SL = SLOTS, bool ONE = false>
+// PK: the reproducible HG walk's instance, whose tail is hg_tail; without it
+// the HG walk has the cooperative tail.  One instance with both spilled 47
+// registers instead of 5.
+template <class W, int WPE, bool DIRECT = false, int SL = SLOTS, bool ONE = false, bool PK = false>
 __global__ void __launch_bounds__(W::MAX_BLOCK) __attribute__((amdgpu_waves_per_eu(WPE)))
 k_walk(const KParams P)
 {
-    constexpr bool HAND = W::COOP && WPE <= 5;
+    constexpr bool HAND = W::COOP && !PK && WPE <= 5;
     __shared__ BlockStateT<SL> bs;
     // native mode: coop_live table entries per wave, then coop_live group slots per wave
     extern __shared__ CoopEntry coop_tab[];
@@ -574,7 +622,15 @@ k_walk(const KParams P)
             if (++spins > (1 << 28)) break;  // cannot happen: chunks always finish
             continue;
         }
-        if constexpr (W::COOP) {
+        if constexpr (PK) {
+            // queue empty and few photons left: the packet tail
+            if (lds_load(&bs.exhausted) && __popcll(live) <= HG_TAIL) {
+                __builtin_amdgcn_s_setprio(3);
+                hg_tail(w, state, P, wave);
+                retire<W, DIRECT>(bs, P, w, state, my_slot, my_gid);
+                break;
+            }
+        } else if constexpr (W::COOP) {
             // queue empty and few photons left: walk them cooperatively
             if (lds_load(&bs.exhausted) && __popcll(live) <= P.coop_live) {
                 if constexpr (HAND) {
@@ -586,17 +642,6 @@ k_walk(const KParams P)
                     retire<W, DIRECT>(bs, P, w, state, my_slot, my_gid);
                 }
                 break;
-            }
-            // reproducible mode (no cooperative tail): the packet tail mode,
-            // in the 128-VGPR build (in the smaller ones its code would add
-            // spills to the step loop; they keep the one-lane drain)
-            if constexpr (HG_TAIL_IN<WPE>) {
-                if (P.coop_live == 0 && lds_load(&bs.exhausted) && __popcll(live) <= HG_TAIL) {
-                    __builtin_amdgcn_s_setprio(3);
-                    hg_tail<WPE>(w, state, P, wave);
-                    retire<W, DIRECT>(bs, P, w, state, my_slot, my_gid);
-                    break;
-                }
             }
         }
         constexpr bool PTAIL = W::STOKES && !W::COOP && sizeof(typename W::Real) == 4;
@@ -613,7 +658,7 @@ k_walk(const KParams P)
         }
         // leave the hot loop once `thresh` lanes are not live (with the queue
         // empty: once the cooperative tail can take over)
-        const int thresh = lds_load(&bs.exhausted) ? (W::COOP ? 64 - tail_live<WPE>(P) : 64 - ptail)
+        const int thresh = lds_load(&bs.exhausted) ? (PK ? 64 - HG_TAIL : W::COOP ? 64 - P.coop_live : 64 - ptail)
                                                    : min(64, (64 - __popcll(live)) + (int)P.refill_min);
         // ---------------- hot: step every live photon
         // Two steps per loop turn, the exit test after the second: the next
@@ -1480,7 +1525,7 @@ static int64_t count_chunks(const mcs_ctx *c, int chunk)
 //   as many blocks as are resident together, the photons spread evenly over
 //   them.  Kernel ms at the default shape (256, 4, 2048, 8), queue -> ONE:
 //   coop_live 0: 2,000 photons 1.50 -> 0.70, 10,000 1.53 -> 0.76, 250,000 1.98
-//   -> 1.54; polarised: 2,000 1.51 -> 0.43, 20,000 1.82 -> 0.77, 100,000 1.96 ->
+//   -> 1.54 (0.36, 0.41 and 1.05 since hg_tail runs in batches); polarised: 2,000 1.51 -> 0.43, 20,000 1.82 -> 0.77, 100,000 1.96 ->
 //   1.02.  Polarised blocks of 512 threads, one per CU, hold the photons up to
 //   8 waves per CU (20,000 photons: 0.77 ms; 256-thread blocks, three per CU,
 //   0.95: three waves share a SIMD from the start, and not evenly), then
@@ -1584,29 +1629,27 @@ static int enqueue_walk(mcs_ctx *c, int mode, const KParams &P, const WalkShape 
         // 6-wave build's spills sit outside the step loop)
         // (ONE is built for 4 and keeps at most that many resident)
         const int waves_per_simd = shape.take > 0 ? 4 : (c->launch.blocks_per_cu * (block / 64) + 3) / 4;
-        // cooperative tables, or at coop_live 0 the packet tail's owners and
-        // packets (in the build that carries it)
-        const size_t tab = c->launch.coop_live > 0
-                               ? (size_t)(block / 64) * c->launch.coop_live * (sizeof(CoopEntry) + sizeof(int))
-                           : waves_per_simd <= 4
-                               ? (size_t)(block / 64) * (HG_TAIL * sizeof(int) + HG_PK_SLOTS * sizeof(HgPacket))
-                               : 0;
-        if (shape.take > 0 && P.rec_direct)
-            hipLaunchKernelGGL((k_walk<NativeWalker, 4, true, SLOTS, true>), dim3(grid), dim3(block), tab, c->stream, P);
+        // cooperative tables, or the packet tail's (the 5- and 6-wave builds
+        // walk one photon per lane to the end at coop_live 0)
+        const bool pk = c->launch.coop_live == 0 && waves_per_simd <= 4;
+        const size_t tab = pk ? (size_t)(block / 64) * sizeof(HgTab)
+                              : (size_t)(block / 64) * c->launch.coop_live * (sizeof(CoopEntry) + sizeof(int));
+        const auto go = [&](auto kernel) {
+            hipLaunchKernelGGL(kernel, dim3(grid), dim3(block), tab, c->stream, P);
+        };
+        const bool direct = P.rec_direct != 0;
+        if (shape.take > 0 && pk)
+            direct ? go(k_walk<NativeWalker, 4, true, SLOTS, true, true>) : go(k_walk<NativeWalker, 4, false, SLOTS, true, true>);
         else if (shape.take > 0)
-            hipLaunchKernelGGL((k_walk<NativeWalker, 4, false, SLOTS, true>), dim3(grid), dim3(block), tab, c->stream, P);
-        else if (waves_per_simd > 5 && P.rec_direct)
-            hipLaunchKernelGGL((k_walk<NativeWalker, 6, true>), dim3(grid), dim3(block), tab, c->stream, P);
-        else if (waves_per_simd > 5)
-            hipLaunchKernelGGL((k_walk<NativeWalker, 6>), dim3(grid), dim3(block), tab, c->stream, P);
-        else if (waves_per_simd <= 4 && P.rec_direct)
-            hipLaunchKernelGGL((k_walk<NativeWalker, 4, true>), dim3(grid), dim3(block), tab, c->stream, P);
+            direct ? go(k_walk<NativeWalker, 4, true, SLOTS, true>) : go(k_walk<NativeWalker, 4, false, SLOTS, true>);
+        else if (pk)
+            direct ? go(k_walk<NativeWalker, 4, true, SLOTS, false, true>) : go(k_walk<NativeWalker, 4, false, SLOTS, false, true>);
         else if (waves_per_simd <= 4)
-            hipLaunchKernelGGL((k_walk<NativeWalker, 4>), dim3(grid), dim3(block), tab, c->stream, P);
-        else if (P.rec_direct)
-            hipLaunchKernelGGL((k_walk<NativeWalker, 5, true>), dim3(grid), dim3(block), tab, c->stream, P);
+            direct ? go(k_walk<NativeWalker, 4, true>) : go(k_walk<NativeWalker, 4>);
+        else if (waves_per_simd == 5)
+            direct ? go(k_walk<NativeWalker, 5, true>) : go(k_walk<NativeWalker, 5>);
         else
-            hipLaunchKernelGGL((k_walk<NativeWalker, 5>), dim3(grid), dim3(block), tab, c->stream, P);
+            direct ? go(k_walk<NativeWalker, 6, true>) : go(k_walk<NativeWalker, 6>);
     } else {
         hipLaunchKernelGGL((k_walk<ReplayWalker, ReplayWalker::WAVES_PER_EU>), dim3(grid), dim3(block), 0,
                            c->stream, P);

@@ -65,15 +65,21 @@ static_assert(sizeof(PolarPacket) == 80, "PolarPacket: five 16-byte LDS loads");
 // The state-independent part of a step of the HG walk: free path, absorption
 // word, cos and sin theta, the azimuth's sine and cosine (hg_packet, from the
 // step's Philox block with the expressions of NativeWalkerT::step, so that a
-// step formed from a packet built in another lane rounds alike).  32 bytes,
-// two 16-byte LDS loads.
-struct alignas(16) HgPacket {
+// step formed from a packet built in another lane rounds alike).
+struct HgPacket {
     float dtau;
     uint32_t w;
     float cost, sint, sinp, cosp;
-    float pad0, pad1;
 };
-static_assert(sizeof(HgPacket) == 32, "HgPacket: two 16-byte LDS loads");
+
+// Steps of the reproducible HG walk's tail between two event tests, and a
+// batch of them: cos and sin theta, sin and cos phi; free paths; each step's
+// vertical cosine before it and sin theta over its horizontal length
+constexpr int HG_BATCH = 4;
+struct HgBatch {
+    float4 r[HG_BATCH], d;
+    float u[HG_BATCH], st[HG_BATCH];
+};
 
 // sin and cos of phi and of 2 phi for 2 phi = r2 revolutions (one
 // transcendental pair; no implicit contraction, so every caller rounds alike)
@@ -454,12 +460,54 @@ struct NativeWalkerT {
         o.sint = __builtin_amdgcn_sqrtf(fmaf(-o.cost, o.cost, 1.f));
         o.sinp = __builtin_amdgcn_sinf(rev);
         o.cosp = __builtin_amdgcn_cosf(rev);
-        o.pad0 = o.pad1 = 0.f;
     }
 
-    // The move of a step from its packet (the expressions of step()); true
-    // when an event follows (exit through either face, or absorbed)
-    __device__ __forceinline__ bool hg_move(const HgPacket &k)
+    // Four steps from their packets (the expressions of step() away from the
+    // vertical) in two parts.  hg_dive: vertical cosine u and depth z through
+    // the steps; keeps each step's u and st = sin theta / sqrt(1 - u^2) for
+    // hg_swing, and returns a value > 0 iff some step leaves the slab (z > 0 or
+    // z < cap) or starts too near the vertical for this form (s2 < 1e-7; the
+    // signs of these differences are exact).  hg_swing: the horizontal cosines
+    // and the optical path through the same.
+    __device__ __forceinline__ static void hg_load(HgBatch &q, const float4 *rot, const float *dt)
+    {
+        for (int m = 0; m < HG_BATCH; ++m) q.r[m] = rot[m];
+        q.d = *reinterpret_cast<const float4 *>(dt);
+    }
+    __device__ __forceinline__ static float hg_dive(HgBatch &q, float &u, float &z, float cap)
+    {
+        const float d[HG_BATCH] = {q.d.x, q.d.y, q.d.z, q.d.w};
+        float zx = 0.f, zn = 0.f, sm = 0.f;
+#pragma unroll
+        for (int m = 0; m < HG_BATCH; ++m) {
+            const float cost = q.r[m].x, sint = q.r[m].y, cosp = q.r[m].w;
+            const float s2 = fmaf(-u, u, 1.f);
+            const float st = sint * __builtin_amdgcn_rsqf(s2);
+            q.u[m] = u;
+            q.st[m] = st;
+            u = fmaf(-s2 * st, cosp, u * cost);
+            z = fmaf(d[m], u, z);
+            zx = m ? fmaxf(zx, z) : z;
+            zn = m ? fminf(zn, z) : z;
+            sm = m ? fminf(sm, s2) : s2;
+        }
+        return fmaxf(fmaxf(zx, cap - zn), 1e-7f - sm);
+    }
+    __device__ __forceinline__ void hg_swing(const HgBatch &q)
+    {
+        const float d[HG_BATCH] = {q.d.x, q.d.y, q.d.z, q.d.w};
+#pragma unroll
+        for (int m = 0; m < HG_BATCH; ++m) {
+            const float cost = q.r[m].x, sinp = q.r[m].z, cosp = q.r[m].w, st = q.st[m], u = q.u[m];
+            const float gx = fmaf(st, fmaf(mux * u, cosp, -muy * sinp), mux * cost);
+            const float gy = fmaf(st, fmaf(muy * u, cosp, mux * sinp), muy * cost);
+            mux = gx; muy = gy;
+            tau_acc += d[m];
+        }
+    }
+
+    // A step from its packet with the axis form and the step count
+    __device__ __forceinline__ void hg_move(const HgPacket &k)
     {
         ++i;
         const float cost = k.cost, sint = k.sint, sinp = k.sinp, cosp = k.cosp;
@@ -480,7 +528,6 @@ struct NativeWalkerT {
         }
         z = fmaf(k.dtau, muz, z);
         tau_acc += k.dtau;
-        return z > 0.f || z < -tau_tot || k.w < t_abs_all;
     }
 
     // ids from the Philox words: ck0 = case ^ k0, l0 = lo(M0 * photon) with
