@@ -8,6 +8,8 @@
 // fused: bias + SiLU (forward, keeping the FP32 pre-activation for the
 // backward pass), SiLU' (backward), a plain FP32 store, or an FP32 atomic add
 // of a split-K partial (weight gradients: few output tiles, K = batch rows).
+// 256-wide networks have kernels of their own: k_mlp_fused (inference) and
+// those of mlp_train.h.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -517,6 +519,8 @@ __global__ void k_adam(float *p, const float *gr, float *m, float *v, const uint
 
 }  // namespace mlp
 
+#include "mlp_train.h"
+
 // =================================================================== host
 using namespace mlp;
 
@@ -548,6 +552,16 @@ struct mcs_mlp {
     int32_t *idx = nullptr;
     float *lpart = nullptr;          // k_loss: per-block partial sums (LOSS_BLOCKS)
     bool fused = false;              // inference through k_mlp_fused
+    // training through k_train_rows / k_train_dw / k_train_adam: 256-wide
+    // networks within its limits.  Their operand copies of the weights, the
+    // per-slice gradient sums; activations and gradients go, transposed, into
+    // X, A, Z (as bf16) and dY.
+    bool train_rows = false;
+    bf16 *wf = nullptr, *wt = nullptr;
+    float *part = nullptr;
+    ParamMap pm{};
+    int32_t *didx = nullptr;         // row indices of a train_steps call (grown on demand)
+    size_t didx_cap = 0;
     float *xd = nullptr, *td = nullptr;
     int64_t n_data = 0;
     double last_ms = 0.0;
@@ -723,6 +737,69 @@ static void backward_pass(mcs_mlp *c, int rows, float *loss_out)
     }
 }
 
+// ---- training of 256-wide networks (mlp_train.h): three kernels a step.  At
+// batch 4096 and 9 -> 4 x 256 -> 651 on MI355X k_train_rows takes 27 us,
+// k_train_dw 10 and k_train_adam 7 (the per-layer kernels, which other widths,
+// deeper or wider-output networks use: 26 launches, 234 us); 48 steps with
+// their uploads 11.2 -> 2.45 ms.
+static void pack_weights(mcs_mlp *c)
+{
+    hipLaunchKernelGGL(k_pack_weights, dim3((unsigned)((c->n_pad + 255) / 256)), dim3(256), 0, c->stream, c->pm, c->p,
+                       c->wb, c->wf, c->wt);
+}
+
+// Partial gradients (c->part, `slices` of them) and per-block loss sums
+// (c->lpart, batch / TR_ROWS) of `batch` rows: idx into x, t (n_data rows), or
+// the first `batch` rows (idx null).
+static int rows_backward(mcs_mlp *c, const float *x, const float *t, int64_t n_data, const int32_t *idx, int batch)
+{
+    const int L = c->d.n_hidden_layers;
+    TrainArgs g;
+    DwArgs d;
+    memset(&g, 0, sizeof g);
+    memset(&d, 0, sizeof d);
+    g.x = x; g.t = t; g.idx = idx; g.n_data = n_data;
+    g.n_in = c->d.n_in; g.n_out = c->d.n_out; g.np = c->np; g.batch = batch;
+    g.ld = batch + LD_PAD;
+    g.p = c->p; g.w = c->w; g.wf = c->wf; g.wt = c->wt;
+    g.xt = c->X; g.dyt = c->dY; g.lpart = c->lpart;
+    // batch slices of the weight gradients: 8, each a multiple of 64 rows
+    d.L = L; d.batch = batch; d.ld = g.ld; d.n_pad = c->n_pad; d.part = c->part;
+    d.kchunk = ((batch + DW_SLICES - 1) / DW_SLICES + 63) / 64 * 64;
+    const int slices = d.slices = (batch + d.kchunk - 1) / d.kchunk;
+    int tiles = 0;
+    for (int l = 0; l <= L; ++l) {
+        const Layer &ly = c->layers[l];
+        g.woff[l] = ly.wb_off; g.boff[l] = ly.b_off;
+        if (l < L) {
+            g.at[l] = c->A[l];
+            g.dzt[l] = reinterpret_cast<bf16 *>(c->Z[l]);
+        }
+        d.tile0[l] = tiles;
+        d.mtiles[l] = ly.prow / 64; d.cols[l] = ly.pcol;
+        d.dz[l] = l < L ? g.dzt[l] : g.dyt;
+        d.in[l] = l ? g.at[l - 1] : g.xt;
+        d.woff[l] = ly.w_off; d.boff[l] = ly.b_off;
+        tiles += d.mtiles[l] * ((ly.pcol + 63) / 64);
+    }
+    d.tile0[L + 1] = tiles;
+    const auto go = [&](auto kernel) {
+        hipLaunchKernelGGL(kernel, dim3(batch / TR_ROWS), dim3(TR_WAVES * 64), 0, c->stream, g);
+    };
+    switch (L) {
+    case 1: go(k_train_rows<1>); break;
+    case 2: go(k_train_rows<2>); break;
+    case 3: go(k_train_rows<3>); break;
+    case 4: go(k_train_rows<4>); break;
+    case 5: go(k_train_rows<5>); break;
+    case 6: go(k_train_rows<6>); break;
+    case 7: go(k_train_rows<7>); break;
+    default: go(k_train_rows<8>); break;
+    }
+    hipLaunchKernelGGL(k_train_dw, dim3(tiles * slices), dim3(256), 0, c->stream, d);
+    return slices;
+}
+
 static int check_dims(const mcs_mlp_dims *d)
 {
     return d && d->n_in >= 1 && d->n_in <= K0 && d->hidden >= 64 && d->hidden % 64 == 0 && d->hidden <= 1024 &&
@@ -752,6 +829,7 @@ int mcs_mlp_create(int device, const mcs_mlp_dims *dims, mcs_mlp **out)
         const char *e = getenv("MCS_MLP_LAYERED");
         c->fused = dims->hidden == FUSED_H && dims->n_hidden_layers <= FUSED_MAX_LAYERS && !(e && e[0] == '1');
     }
+    c->train_rows = c->fused && dims->hidden == TR_H && dims->n_hidden_layers <= TR_MAX_LAYERS && c->np <= TR_MAX_NP;
     if (hipSetDevice(device) != hipSuccess || hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking) != hipSuccess ||
         hipEventCreate(&c->e0) != hipSuccess || hipEventCreate(&c->e1) != hipSuccess) {
         mcs_mlp_destroy(c);
@@ -788,19 +866,31 @@ int mcs_mlp_create(int device, const mcs_mlp_dims *dims, mcs_mlp **out)
     bool ok = dalloc(&c->p, off) == hipSuccess && dalloc(&c->gr, off) == hipSuccess &&
               dalloc(&c->m, off) == hipSuccess && dalloc(&c->v, off) == hipSuccess &&
               dalloc(&c->mask, off) == hipSuccess && dalloc(&c->pb_index, off) == hipSuccess &&
-              dalloc(&c->wb, woff) == hipSuccess && dalloc(&c->X, MB * K0) == hipSuccess &&
-              dalloc(&c->dY, MB * c->np) == hipSuccess && dalloc(&c->dZa, MB * H) == hipSuccess &&
+              dalloc(&c->wb, woff) == hipSuccess && dalloc(&c->X, (MB + LD_PAD) * K0) == hipSuccess &&
+              dalloc(&c->dY, (MB + LD_PAD) * c->np) == hipSuccess && dalloc(&c->dZa, MB * H) == hipSuccess &&
               dalloc(&c->dZb, MB * H) == hipSuccess && dalloc(&c->Y, MB * c->np) == hipSuccess &&
               dalloc(&c->T, MB * c->np) == hipSuccess && dalloc(&c->w, c->np) == hipSuccess &&
               dalloc(&c->yout, MB * dims->n_out) == hipSuccess && dalloc(&c->xin, MB * dims->n_in) == hipSuccess &&
               dalloc(&c->loss, 1024) == hipSuccess && dalloc(&c->idx, MB) == hipSuccess &&
-              dalloc(&c->lpart, LOSS_BLOCKS) == hipSuccess;
+              dalloc(&c->lpart, std::max<size_t>(LOSS_BLOCKS, MB / TR_ROWS)) == hipSuccess;
     for (int l = 0; ok && l < L; ++l) {
         float *z = nullptr;
         bf16 *a = nullptr;
-        ok = dalloc(&z, MB * H) == hipSuccess && dalloc(&a, MB * H) == hipSuccess;
+        ok = dalloc(&z, MB * H) == hipSuccess && dalloc(&a, (MB + LD_PAD) * H) == hipSuccess;
         c->Z.push_back(z);
         c->A.push_back(a);
+    }
+    if (ok && c->train_rows) {
+        ok = dalloc(&c->wf, woff) == hipSuccess && dalloc(&c->wt, woff) == hipSuccess &&
+             dalloc(&c->part, DW_SLICES * off) == hipSuccess;
+        c->pm.L = L;
+        c->pm.n_pad = off;
+        for (int l = 0; l <= L; ++l) {
+            const Layer &ly = c->layers[l];
+            c->pm.woff[l] = ly.w_off; c->pm.boff[l] = ly.b_off; c->pm.wboff[l] = ly.wb_off;
+            c->pm.rows[l] = ly.rows; c->pm.cols[l] = ly.cols; c->pm.prow[l] = ly.prow;
+            c->pm.lgcol[l] = ly.pcol == K0 ? 5 : 8;
+        }
     }
     if (!ok) {
         mcs_mlp_destroy(c);
@@ -825,7 +915,7 @@ int mcs_mlp_destroy(mcs_mlp *c)
     if (c->stream) (void)hipStreamSynchronize(c->stream);
     void *bufs[] = {c->p, c->gr, c->m, c->v, c->mask, c->pb_index, c->wb, c->X, c->dY, c->dZa, c->dZb,
                     c->Y, c->T, c->w, c->yout, c->xin, c->loss, c->idx, c->xd, c->td,
-                    c->fmu, c->fsd, c->oscale, c->oshift, c->ooff, c->lpart};
+                    c->fmu, c->fsd, c->oscale, c->oshift, c->ooff, c->lpart, c->wf, c->wt, c->part, c->didx};
     for (void *b : bufs) if (b) (void)hipFree(b);
     for (float *z : c->Z) if (z) (void)hipFree(z);
     for (bf16 *a : c->A) if (a) (void)hipFree(a);
@@ -868,6 +958,11 @@ int mcs_mlp_set_params(mcs_mlp *c, const float *params, int64_t n)
     MCHK(c, hipMemcpy(c->wb, wb.data(), wb.size() * 2, hipMemcpyHostToDevice));
     MCHK(c, hipMemset(c->m, 0, c->n_pad * 4));
     MCHK(c, hipMemset(c->v, 0, c->n_pad * 4));
+    if (c->train_rows) {
+        pack_weights(c);
+        MCHK(c, hipGetLastError());
+        MCHK(c, hipStreamSynchronize(c->stream));
+    }
     return MCS_OK;
 }
 
@@ -1013,6 +1108,17 @@ static int upload_weights(mcs_mlp *c, const float *w)
     return MCS_OK;
 }
 
+static int finish_grads(mcs_mlp *c, float *grads, float *loss)
+{
+    MCHK(c, hipGetLastError());
+    MCHK(c, hipStreamSynchronize(c->stream));
+    std::vector<float> pad(c->n_pad);
+    MCHK(c, hipMemcpy(pad.data(), c->gr, pad.size() * 4, hipMemcpyDeviceToHost));
+    unpad(c, pad, grads);
+    if (loss) MCHK(c, hipMemcpy(loss, c->loss, 4, hipMemcpyDeviceToHost));
+    return MCS_OK;
+}
+
 int mcs_mlp_grads(mcs_mlp *c, const float *x, const float *t, const float *w, int32_t n, float *grads, float *loss)
 {
     if (!c || !x || !t || !w || !grads) return MCS_ERR_ARG;
@@ -1021,6 +1127,14 @@ int mcs_mlp_grads(mcs_mlp *c, const float *x, const float *t, const float *w, in
     int r = upload_weights(c, w);
     if (r) return r;
     const int ni = c->d.n_in, no = c->d.n_out;
+    if (c->train_rows) {
+        MCHK(c, hipMemcpy(c->xin, x, sizeof(float) * n * ni, hipMemcpyHostToDevice));
+        MCHK(c, hipMemcpy(c->T, t, sizeof(float) * n * no, hipMemcpyHostToDevice));
+        const int slices = rows_backward(c, c->xin, c->T, n, nullptr, n);
+        hipLaunchKernelGGL(k_train_reduce, dim3((unsigned)((c->n_pad + 255) / 256)), dim3(256), 0, c->stream, c->pm,
+                           c->part, slices, c->gr, c->lpart, n / TR_ROWS, n, c->loss);
+        return finish_grads(c, grads, loss);
+    }
     std::vector<float> tp((size_t)n * c->np, 0.f);
     for (int i = 0; i < n; ++i)
         for (int k = 0; k < no; ++k) tp[(size_t)i * c->np + k] = t[(size_t)i * no + k];
@@ -1029,13 +1143,7 @@ int mcs_mlp_grads(mcs_mlp *c, const float *x, const float *t, const float *w, in
     hipLaunchKernelGGL(k_cast_x, dim3((n * K0 + 255) / 256), dim3(256), 0, c->stream, c->xin, ni, n, c->X);
     forward_pass(c, n);
     backward_pass(c, n, c->loss);
-    MCHK(c, hipGetLastError());
-    MCHK(c, hipStreamSynchronize(c->stream));
-    std::vector<float> pad(c->n_pad);
-    MCHK(c, hipMemcpy(pad.data(), c->gr, pad.size() * 4, hipMemcpyDeviceToHost));
-    unpad(c, pad, grads);
-    if (loss) MCHK(c, hipMemcpy(loss, c->loss, 4, hipMemcpyDeviceToHost));
-    return MCS_OK;
+    return finish_grads(c, grads, loss);
 }
 
 int mcs_mlp_set_dataset(mcs_mlp *c, const float *x, const float *t, int64_t n)
@@ -1067,24 +1175,57 @@ int mcs_mlp_train_steps(mcs_mlp *c, const int32_t *idx, int32_t n_steps, int32_t
     (void)hipSetDevice(c->device);
     int r = upload_weights(c, w);
     if (r) return r;
-    int32_t *didx = nullptr;
-    MCHK(c, dalloc(&didx, (size_t)n_steps * batch));
-    hipError_t e = hipMemcpy(didx, idx, sizeof(int32_t) * (size_t)n_steps * batch, hipMemcpyHostToDevice);
-    if (e != hipSuccess) { (void)hipFree(didx); return merr(c, MCS_ERR_HIP, "idx upload: %s", hipGetErrorString(e)); }
+    const size_t ni = (size_t)n_steps * batch;
+    if (ni > c->didx_cap) {
+        if (c->didx) { (void)hipFree(c->didx); c->didx = nullptr; c->didx_cap = 0; }
+        MCHK(c, dalloc(&c->didx, ni));
+        c->didx_cap = ni;
+    }
+    MCHK(c, hipMemcpy(c->didx, idx, sizeof(int32_t) * ni, hipMemcpyHostToDevice));
+    AdamArgs adam;
+    memset(&adam, 0, sizeof adam);
+    int adam_blocks = 0;
+    if (c->train_rows) {
+        adam.m = c->pm;
+        adam.part = c->part;
+        adam.p = c->p; adam.mo = c->m; adam.vo = c->v;
+        adam.b1 = a->beta1; adam.b2 = a->beta2; adam.eps = a->eps; adam.wd_lr = a->lr * a->weight_decay;
+        adam.wf = c->wf; adam.wt = c->wt;
+        adam.lpart = c->lpart; adam.nb = batch / TR_ROWS; adam.rows = batch;
+        int patches = 0, bias = 0;
+        for (size_t l = 0; l < c->layers.size(); ++l) {
+            adam.patch0[l] = patches;
+            adam.bias0[l] = bias;
+            patches += (c->layers[l].prow / 32) * (c->layers[l].pcol / 32);
+            bias += (c->layers[l].rows + 255) / 256;
+        }
+        adam.patch0[c->layers.size()] = patches;
+        adam.bias0[c->layers.size()] = bias;
+        adam_blocks = patches + bias;
+    }
     for (int s = 0; s < n_steps; ++s) {
-        hipLaunchKernelGGL(k_gather, dim3(batch), dim3(64), 0, c->stream, c->xd, c->td, didx + (size_t)s * batch,
-                           c->d.n_in, c->d.n_out, c->np, batch, c->n_data, c->X, c->T);
-        forward_pass(c, batch);
-        backward_pass(c, batch, c->loss + 1 + s);   // step s's loss in loss[1 + s]
+        const int32_t *rows = c->didx + (size_t)s * batch;
+        float *const loss_out = c->loss + 1 + s;   // step s's loss in loss[1 + s]
         const int t = a->step + s + 1;
         const float lr_t = a->lr * std::sqrt(1.f - std::pow(a->beta2, (float)t)) / (1.f - std::pow(a->beta1, (float)t));
+        if (c->train_rows) {
+            const int slices = rows_backward(c, c->xd, c->td, c->n_data, rows, batch);
+            adam.slices = slices;
+            adam.lr_t = lr_t;
+            adam.loss = loss_out;
+            hipLaunchKernelGGL(k_train_adam, dim3(adam_blocks), dim3(256), 0, c->stream, adam);
+            continue;
+        }
+        hipLaunchKernelGGL(k_gather, dim3(batch), dim3(64), 0, c->stream, c->xd, c->td, rows,
+                           c->d.n_in, c->d.n_out, c->np, batch, c->n_data, c->X, c->T);
+        forward_pass(c, batch);
+        backward_pass(c, batch, loss_out);
         hipLaunchKernelGGL(k_adam, dim3(1024), dim3(256), 0, c->stream, c->p, c->gr, c->m, c->v, c->mask, c->n_pad,
                            lr_t, a->beta1, a->beta2, a->eps, a->lr * a->weight_decay, c->wb, c->pb_index);
     }
-    e = hipGetLastError();
-    if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
-    (void)hipFree(didx);
-    if (e != hipSuccess) return merr(c, MCS_ERR_HIP, "train: %s", hipGetErrorString(e));
+    if (c->train_rows) pack_weights(c);   // the row-major copies inference reads
+    MCHK(c, hipGetLastError());
+    MCHK(c, hipStreamSynchronize(c->stream));
     if (losses) MCHK(c, hipMemcpy(losses, c->loss + 1, sizeof(float) * n_steps, hipMemcpyDeviceToHost));
     return MCS_OK;
 }
