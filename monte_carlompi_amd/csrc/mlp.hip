@@ -8,8 +8,8 @@
 // fused: bias + SiLU (forward, keeping the FP32 pre-activation for the
 // backward pass), SiLU' (backward), a plain FP32 store, or an FP32 atomic add
 // of a split-K partial (weight gradients: few output tiles, K = batch rows).
-// 256-wide networks have kernels of their own: k_mlp_fused (inference) and
-// those of mlp_train.h.
+// 256-wide networks have kernels of their own: mlp_serve.h (inference) and
+// mlp_train.h.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -242,127 +242,6 @@ __global__ void __launch_bounds__(256) k_gemm_fwd(const GemmArgs g)
     }
 }
 
-// ---------------------------------------------------------------- fused
-// The whole network for 128 rows per block: input (K0 = 32 columns) -> L
-// hidden layers of 256 (bias + SiLU, BF16 activations kept in LDS) -> output
-// layer with the F32 or exp epilogue straight to HBM.  Weights (0.8 MB for
-// the surrogate) are read from L2 as MFMA operands, no LDS staging; each of
-// the 8 waves owns one column tile of 32 of a hidden layer (and every 8th
-// of the output layer) and multiplies each weight operand into the block's
-// four 32-row quarters, so the weight traffic per row is a quarter of that
-// of 32-row blocks.  A hidden layer's tiles are computed into registers,
-// then, after a barrier, written over its input (one activation buffer).
-// Built for 2 waves per SIMD (up to 256 VGPRs: the four accumulators and
-// the epilogue without spills).  Measured on MI355X for 1e6 queries: 2.2 ms
-// (3.8 ms with the per-layer kernels; 2.3 ms with 64-row blocks, 3.4 ms
-// with 32-row blocks).  Operands, k order and epilogues are those of
-// k_gemm_fwd, so the results are the same.
-constexpr int FUSED_ROWS = 128, FUSED_Q = FUSED_ROWS / 32, FUSED_WAVES = 8, FUSED_H = 256,
-              FUSED_MAX_LAYERS = 16;
-static_assert(FUSED_H / 32 == FUSED_WAVES, "one hidden column tile per wave");
-struct FusedArgs {
-    const bf16 *X;            // [rows][K0]
-    int rows, L, n_out, np;
-    const bf16 *wb;           // bf16 weights, layer l at woff[l], [prow][pcol]
-    const float *p;           // fp32 parameters (biases at boff[l])
-    size_t woff[FUSED_MAX_LAYERS + 1], boff[FUSED_MAX_LAYERS + 1];
-    float *y;                 // [rows][n_out]
-    const float *oscale, *oshift, *ooff;   // exp epilogue (nullptr: F32)
-};
-
-// acc[q] += A[32 q .. 32 q + 32)[KIN] (LDS, row pitch lda) . W[n0 .. n0 + 32)[KIN]^T
-template <int KIN>
-__device__ __forceinline__ void fused_tile(f32x16 (&acc)[FUSED_Q], const bf16 *A, int lda, const bf16 *W, int n0,
-                                           int lane)
-{
-    const bf16 *wrow = W + (size_t)(n0 + (lane & 31)) * KIN + (lane >> 5) * 8;
-    const bf16 *arow = A + (lane & 31) * lda + (lane >> 5) * 8;
-    // weight operands in groups of up to 4 k-steps
-    constexpr int NS = KIN / 16, GS = NS < 4 ? NS : 4;
-#pragma unroll 1
-    for (int g0 = 0; g0 < NS; g0 += GS) {
-        bf16x8 b[GS];
-#pragma unroll
-        for (int i = 0; i < GS; ++i) b[i] = *reinterpret_cast<const bf16x8 *>(wrow + (g0 + i) * 16);
-#pragma unroll
-        for (int i = 0; i < GS; ++i) {
-            const int k = (g0 + i) * 16;
-#pragma unroll
-            for (int q = 0; q < FUSED_Q; ++q) {
-                const bf16x8 a = *reinterpret_cast<const bf16x8 *>(arow + 32 * q * lda + k);
-                acc[q] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b[i], acc[q], 0, 0, 0);
-            }
-        }
-    }
-}
-
-__global__ void __launch_bounds__(FUSED_WAVES * 64) __attribute__((amdgpu_waves_per_eu(2)))
-k_mlp_fused(const FusedArgs g)
-{
-    constexpr int P0 = K0 + 8, PH = FUSED_H + 8;   // LDS row pitches (bf16)
-    __shared__ __attribute__((aligned(16))) bf16 X0[FUSED_ROWS][P0];
-    __shared__ __attribute__((aligned(16))) bf16 Act[FUSED_ROWS][PH];
-    const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
-    const int r0 = blockIdx.x * FUSED_ROWS;
-    // input rows (zero beyond the last row)
-    for (int i = t; i < FUSED_ROWS * K0 / 8; i += blockDim.x) {
-        const int r = i / (K0 / 8), c8 = (i % (K0 / 8)) * 8;
-        uint4 v = make_uint4(0, 0, 0, 0);
-        if (r0 + r < g.rows) v = *reinterpret_cast<const uint4 *>(g.X + (size_t)(r0 + r) * K0 + c8);
-        *reinterpret_cast<uint4 *>(&X0[r][c8]) = v;
-    }
-    __syncthreads();
-    const int n = wave * 32 + (lane & 31);
-    for (int l = 0; l < g.L; ++l) {
-        f32x16 acc[FUSED_Q];
-#pragma unroll
-        for (int q = 0; q < FUSED_Q; ++q)
-#pragma unroll
-            for (int r = 0; r < 16; ++r) acc[q][r] = 0.f;
-        const bf16 *W = g.wb + g.woff[l];
-        if (l == 0) fused_tile<K0>(acc, &X0[0][0], P0, W, wave * 32, lane);
-        else fused_tile<FUSED_H>(acc, &Act[0][0], PH, W, wave * 32, lane);
-        const float bn = g.p[g.boff[l] + n];
-        __syncthreads();   // every wave has read this layer's input
-#pragma unroll
-        for (int q = 0; q < FUSED_Q; ++q) {
-#pragma unroll
-            for (int r = 0; r < 16; ++r) {
-                const int m = 32 * q + (r >> 2) * 8 + (lane >> 5) * 4 + (r & 3);
-                const float v = acc[q][r] + bn;
-                Act[m][n] = (bf16)(v * sigm(v));
-            }
-        }
-        __syncthreads();
-    }
-    // output layer: np / 32 column tiles over the waves
-    const bf16 *W = g.wb + g.woff[g.L];
-    const float *bias = g.p + g.boff[g.L];
-    for (int nt = wave; nt < g.np / 32; nt += FUSED_WAVES) {
-        f32x16 acc[FUSED_Q];
-#pragma unroll
-        for (int q = 0; q < FUSED_Q; ++q)
-#pragma unroll
-            for (int r = 0; r < 16; ++r) acc[q][r] = 0.f;
-        fused_tile<FUSED_H>(acc, &Act[0][0], PH, W, nt * 32, lane);
-        const int no = nt * 32 + (lane & 31);
-        if (no >= g.n_out) continue;
-        const float bo = bias[no];
-        float osc = 1.f, osh = 0.f, oof = 0.f;
-        if (g.oscale) { osc = g.oscale[no]; osh = g.oshift[no]; oof = g.ooff[no]; }
-#pragma unroll
-        for (int q = 0; q < FUSED_Q; ++q) {
-#pragma unroll
-            for (int r = 0; r < 16; ++r) {
-                const int m = r0 + 32 * q + (r >> 2) * 8 + (lane >> 5) * 4 + (r & 3);
-                if (m >= g.rows) continue;
-                const float v = acc[q][r] + bo;
-                g.y[(size_t)m * g.n_out + no] = g.oscale ? __builtin_amdgcn_exp2f(fmaf(osc, v, osh)) - oof : v;
-            }
-        }
-    }
-}
-
 // X rows (fp32, n_in wide) -> bf16 [rows][K0], zero padded
 __global__ void k_cast_x(const float *x, int n_in, int rows, bf16 *X)
 {
@@ -378,26 +257,41 @@ __global__ void k_cast_x(const float *x, int n_in, int rows, bf16 *X)
 //   sqrt((1 - omega) / (1 - omega g)), log10(tau (1 - omega g)), log10(tau / mu0)
 // each standardised as (f - mu_k) / sd_k, zero padded to K0 columns, bf16.
 constexpr int SNOW_FEATURES = 9;
+struct SnowInputs {
+    double reff, om, g, tau, mu0;
+};
+__device__ __forceinline__ SnowInputs snow_inputs(const float *q)
+{
+    SnowInputs s;
+    s.reff = q[0]; s.om = q[1]; s.g = q[2]; s.tau = q[4];
+    s.mu0 = cos((double)q[3] * (3.141592653589793 / 180.0));
+    return s;
+}
+__device__ __forceinline__ float snow_feature(const SnowInputs &s, int k, const float *mu, const float *sd)
+{
+    // the standardisation in every branch, beside the feature it may be
+    // contracted with: every caller then rounds alike
+    const double m = mu[k], d = sd[k];
+    switch (k) {
+    case 0: return (float)((log(s.reff) - m) / d);
+    case 1: return (float)((log10(fmax(1.0 - s.om, 1e-12)) - m) / d);
+    case 2: return (float)((s.g - m) / d);
+    case 3: return (float)((s.mu0 - m) / d);
+    case 4: return (float)((log10(s.tau) - m) / d);
+    case 5: return (float)((exp(-s.tau / s.mu0) - m) / d);
+    case 6: return (float)((sqrt((1.0 - s.om) / (1.0 - s.om * s.g)) - m) / d);
+    case 7: return (float)((log10(s.tau * (1.0 - s.om * s.g)) - m) / d);
+    default: return (float)((log10(s.tau / s.mu0) - m) / d);
+    }
+}
 __global__ void k_features_snow(const float *in, int rows, const float *mu, const float *sd, bf16 *X)
 {
     const int r = blockIdx.x * blockDim.x + threadIdx.x;
     if (r >= rows) return;
-    const float *q = in + (size_t)r * 5;
-    const double reff = q[0], om = q[1], g = q[2], th = q[3], tau = q[4];
-    const double mu0 = cos(th * (3.141592653589793 / 180.0));
-    double f[SNOW_FEATURES];
-    f[0] = log(reff);
-    f[1] = log10(fmax(1.0 - om, 1e-12));
-    f[2] = g;
-    f[3] = mu0;
-    f[4] = log10(tau);
-    f[5] = exp(-tau / mu0);
-    f[6] = sqrt((1.0 - om) / (1.0 - om * g));
-    f[7] = log10(tau * (1.0 - om * g));
-    f[8] = log10(tau / mu0);
+    const SnowInputs s = snow_inputs(in + (size_t)r * 5);
     bf16 *row = X + (size_t)r * K0;
-    for (int k = 0; k < K0; ++k)
-        row[k] = (bf16)(k < SNOW_FEATURES ? (float)((f[k] - (double)mu[k]) / (double)sd[k]) : 0.f);
+#pragma unroll
+    for (int k = 0; k < K0; ++k) row[k] = (bf16)(k < SNOW_FEATURES ? snow_feature(s, k, mu, sd) : 0.f);
 }
 
 // minibatch gather from the resident dataset
@@ -519,6 +413,7 @@ __global__ void k_adam(float *p, const float *gr, float *m, float *v, const uint
 
 }  // namespace mlp
 
+#include "mlp_serve.h"
 #include "mlp_train.h"
 
 // =================================================================== host
@@ -551,7 +446,10 @@ struct mcs_mlp {
     float *Y = nullptr, *T = nullptr, *w = nullptr, *yout = nullptr, *xin = nullptr, *loss = nullptr;
     int32_t *idx = nullptr;
     float *lpart = nullptr;          // k_loss: per-block partial sums (LOSS_BLOCKS)
-    bool fused = false;              // inference through k_mlp_fused
+    // inference through k_mlp_serve (256-wide networks) and its operand copy of
+    // the weights
+    bool fused = false;
+    bf16 *ws = nullptr;
     // training through k_train_rows / k_train_dw / k_train_adam: 256-wide
     // networks within its limits.  Their operand copies of the weights, the
     // per-slice gradient sums; activations and gradients go, transposed, into
@@ -630,21 +528,61 @@ static void gemm_fwd(mcs_mlp *c, const GemmArgs &g)
     hipLaunchKernelGGL((k_gemm_fwd<EPI>), grid, dim3(256), 0, c->stream, g);
 }
 
-// inference of `rows` rows already in c->X; outputs [rows][n_out] into `y`
-// (through the output transform when `exp_out`)
+// Inference of a 256-wide network, any number of rows in one launch: x device
+// rows (raw case inputs if `snow`, else n_in features), outputs [rows][n_out]
+// into `y` (through the output transform if `exp_out`).  Rows per block: 128
+// where that fills the CUs twice (operands from L2 and LDS are then shared by
+// the most rows), 64 up to two such blocks per CU, 32 up to one per CU: small
+// batches then spread over more CUs, and what they take is mostly the 0.75 MB of
+// weights through one CU (64 B a cycle).  Measured on MI355X, device us with 32
+// / 64 / 128 rows: 301 rows 20 / 24 / 37, 8,193 rows 40 / 29 / 41, 32,768 rows
+// 83 / 51 / 54, 65,536 rows - / 102 / 90, 1e6 rows - / 1361 / 1267 (the kernel
+// before, 128 rows in 512-thread blocks of one per CU after a feature kernel,
+// in passes of max_batch rows: 65, 69, 75, 139 and 2112).
+static void serve_rows(mcs_mlp *c, const float *x, int64_t rows, float *y, bool snow, bool exp_out)
+{
+    ServeArgs g;
+    memset(&g, 0, sizeof g);
+    g.x = x; g.rows = rows; g.snow = snow; g.n_in = c->d.n_in;
+    g.L = c->d.n_hidden_layers; g.n_out = c->d.n_out; g.np = c->np;
+    g.fmu = c->fmu; g.fsd = c->fsd;
+    g.w = c->ws; g.p = c->p; g.y = y;
+    for (int l = 0; l <= g.L; ++l) { g.woff[l] = c->layers[l].wb_off; g.boff[l] = c->layers[l].b_off; }
+    if (exp_out) { g.oscale = c->oscale; g.oshift = c->oshift; g.ooff = c->ooff; }
+    const auto go = [&](auto kernel, int R) {
+        hipLaunchKernelGGL(kernel, dim3((unsigned)((rows + R - 1) / R)), dim3(SV_WAVES * 64), 0, c->stream, g);
+    };
+    if (rows <= 32 * 256)
+        exp_out ? go(k_mlp_serve<1, 16, 2, true>, 32) : go(k_mlp_serve<1, 16, 2, false>, 32);
+    else if (rows <= 64 * 512)
+        exp_out ? go(k_mlp_serve<2, 4, 4, true>, 64) : go(k_mlp_serve<2, 4, 4, false>, 64);
+    else
+        exp_out ? go(k_mlp_serve<4, 4, 4, true>, 128) : go(k_mlp_serve<4, 4, 4, false>, 128);
+}
+
+// the weights' operand copies from the FP32 parameters
+static void pack_serve(mcs_mlp *c)
+{
+    ServePack s;
+    memset(&s, 0, sizeof s);
+    s.L = c->d.n_hidden_layers;
+    int blocks = 0;
+    for (int l = 0; l <= s.L; ++l) {
+        const Layer &ly = c->layers[l];
+        s.poff[l] = ly.w_off; s.woff[l] = ly.wb_off; s.prow[l] = ly.prow;
+        s.lgcol[l] = ly.pcol == K0 ? 5 : 8;
+        s.block0[l] = blocks;
+        blocks += ly.prow * ly.pcol / 256;
+    }
+    s.block0[s.L + 1] = blocks;
+    hipLaunchKernelGGL(k_pack_serve, dim3(blocks), dim3(256), 0, c->stream, s, c->p, c->ws);
+}
+
+// inference of `rows` rows already in c->X through the per-layer kernels;
+// outputs [rows][n_out] into `y` (through the output transform when `exp_out`)
 static void infer_pass(mcs_mlp *c, int rows, float *y, bool exp_out = false)
 {
     const int L = c->d.n_hidden_layers;
-    if (c->fused) {
-        FusedArgs f;
-        memset(&f, 0, sizeof f);
-        f.X = c->X; f.rows = rows; f.L = L; f.n_out = c->d.n_out; f.np = c->np;
-        f.wb = c->wb; f.p = c->p; f.y = y;
-        for (int l = 0; l <= L; ++l) { f.woff[l] = c->layers[l].wb_off; f.boff[l] = c->layers[l].b_off; }
-        if (exp_out) { f.oscale = c->oscale; f.oshift = c->oshift; f.ooff = c->ooff; }
-        hipLaunchKernelGGL(k_mlp_fused, dim3((rows + FUSED_ROWS - 1) / FUSED_ROWS), dim3(FUSED_WAVES * 64), 0, c->stream, f);
-        return;
-    }
     const bf16 *in = c->X;
     int ld_in = K0;
     for (int l = 0; l < L; ++l) {
@@ -822,12 +760,12 @@ int mcs_mlp_create(int device, const mcs_mlp_dims *dims, mcs_mlp **out)
     c->device = device;
     c->d = *dims;
     c->np = (dims->n_out + 63) / 64 * 64;
-    // inference of 256-wide networks runs fused (k_mlp_fused); the
+    // 256-wide networks run through kernels of their own (k_mlp_serve, mlp_train.h); the
     // environment variable MCS_MLP_LAYERED=1 keeps the per-layer kernels
     // (the same results, for comparison)
     {
         const char *e = getenv("MCS_MLP_LAYERED");
-        c->fused = dims->hidden == FUSED_H && dims->n_hidden_layers <= FUSED_MAX_LAYERS && !(e && e[0] == '1');
+        c->fused = dims->hidden == SV_H && dims->n_hidden_layers <= SV_MAX_LAYERS && !(e && e[0] == '1');
     }
     c->train_rows = c->fused && dims->hidden == TR_H && dims->n_hidden_layers <= TR_MAX_LAYERS && c->np <= TR_MAX_NP;
     if (hipSetDevice(device) != hipSuccess || hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking) != hipSuccess ||
@@ -880,6 +818,7 @@ int mcs_mlp_create(int device, const mcs_mlp_dims *dims, mcs_mlp **out)
         c->Z.push_back(z);
         c->A.push_back(a);
     }
+    if (ok && c->fused) ok = dalloc(&c->ws, woff) == hipSuccess;
     if (ok && c->train_rows) {
         ok = dalloc(&c->wf, woff) == hipSuccess && dalloc(&c->wt, woff) == hipSuccess &&
              dalloc(&c->part, DW_SLICES * off) == hipSuccess;
@@ -915,7 +854,7 @@ int mcs_mlp_destroy(mcs_mlp *c)
     if (c->stream) (void)hipStreamSynchronize(c->stream);
     void *bufs[] = {c->p, c->gr, c->m, c->v, c->mask, c->pb_index, c->wb, c->X, c->dY, c->dZa, c->dZb,
                     c->Y, c->T, c->w, c->yout, c->xin, c->loss, c->idx, c->xd, c->td,
-                    c->fmu, c->fsd, c->oscale, c->oshift, c->ooff, c->lpart, c->wf, c->wt, c->part, c->didx};
+                    c->fmu, c->fsd, c->oscale, c->oshift, c->ooff, c->lpart, c->ws, c->wf, c->wt, c->part, c->didx};
     for (void *b : bufs) if (b) (void)hipFree(b);
     for (float *z : c->Z) if (z) (void)hipFree(z);
     for (bf16 *a : c->A) if (a) (void)hipFree(a);
@@ -958,11 +897,10 @@ int mcs_mlp_set_params(mcs_mlp *c, const float *params, int64_t n)
     MCHK(c, hipMemcpy(c->wb, wb.data(), wb.size() * 2, hipMemcpyHostToDevice));
     MCHK(c, hipMemset(c->m, 0, c->n_pad * 4));
     MCHK(c, hipMemset(c->v, 0, c->n_pad * 4));
-    if (c->train_rows) {
-        pack_weights(c);
-        MCHK(c, hipGetLastError());
-        MCHK(c, hipStreamSynchronize(c->stream));
-    }
+    if (c->train_rows) pack_weights(c);
+    if (c->fused) pack_serve(c);
+    MCHK(c, hipGetLastError());
+    MCHK(c, hipStreamSynchronize(c->stream));
     return MCS_OK;
 }
 
@@ -997,8 +935,12 @@ int mcs_mlp_forward(mcs_mlp *c, const float *x, int64_t n, float *y)
         const int rows = (int)std::min<int64_t>(MB, n - s);
         MCHK(c, hipMemcpyAsync(c->xin, x + s * ni, sizeof(float) * rows * ni, hipMemcpyHostToDevice, c->stream));
         MCHK(c, hipEventRecord(c->e0, c->stream));
-        hipLaunchKernelGGL(k_cast_x, dim3((rows * K0 + 255) / 256), dim3(256), 0, c->stream, c->xin, ni, rows, c->X);
-        infer_pass(c, rows, c->yout);
+        if (c->fused) {
+            serve_rows(c, c->xin, rows, c->yout, false, false);
+        } else {
+            hipLaunchKernelGGL(k_cast_x, dim3((rows * K0 + 255) / 256), dim3(256), 0, c->stream, c->xin, ni, rows, c->X);
+            infer_pass(c, rows, c->yout);
+        }
         MCHK(c, hipEventRecord(c->e1, c->stream));
         MCHK(c, hipGetLastError());
         MCHK(c, hipMemcpyAsync(y + s * no, c->yout, sizeof(float) * rows * no, hipMemcpyDeviceToHost, c->stream));
@@ -1070,7 +1012,8 @@ int mcs_mlp_serve(mcs_mlp *c, const float *d_in, int64_t n, float *d_out)
     const int MB = c->d.max_batch, no = c->d.n_out;
     const int ni = c->feature_map == MCS_FEATURES_SNOW_BRF ? 5 : c->d.n_in;
     MCHK(c, hipEventRecord(c->e0, c->stream));
-    for (int64_t s = 0; s < n; s += MB) {
+    if (c->fused && n > 0) serve_rows(c, d_in, n, d_out, c->feature_map == MCS_FEATURES_SNOW_BRF, true);
+    for (int64_t s = 0; s < n && !c->fused; s += MB) {
         const int rows = (int)std::min<int64_t>(MB, n - s);
         if (c->feature_map == MCS_FEATURES_SNOW_BRF)
             hipLaunchKernelGGL(k_features_snow, dim3((rows + 255) / 256), dim3(256), 0, c->stream, d_in + s * ni, rows,
@@ -1223,7 +1166,7 @@ int mcs_mlp_train_steps(mcs_mlp *c, const int32_t *idx, int32_t n_steps, int32_t
         hipLaunchKernelGGL(k_adam, dim3(1024), dim3(256), 0, c->stream, c->p, c->gr, c->m, c->v, c->mask, c->n_pad,
                            lr_t, a->beta1, a->beta2, a->eps, a->lr * a->weight_decay, c->wb, c->pb_index);
     }
-    if (c->train_rows) pack_weights(c);   // the row-major copies inference reads
+    if (c->fused) pack_serve(c);          // the copy that inference reads
     MCHK(c, hipGetLastError());
     MCHK(c, hipStreamSynchronize(c->stream));
     if (losses) MCHK(c, hipMemcpy(losses, c->loss + 1, sizeof(float) * n_steps, hipMemcpyDeviceToHost));
