@@ -129,11 +129,11 @@ typedef struct {
                                   to enter the cooperative tail once it is
                                   dry).  Walks of fewer photons than the
                                   shape's blocks have chunks for spread them
-                                  over more, smaller chunks, and native walks
-                                  with a lane for every photon deal them out
-                                  once, evenly over the chip (not in the
-                                  cooperative mode above coop_live photons a
-                                  wave).  mcs_get_launch returns the value set */
+                                  over more, smaller chunks, and walks with a
+                                  lane for every photon deal them out once,
+                                  evenly over the chip (not replays of
+                                  aspherical grains, and not the cooperative
+                                  mode above coop_live photons a wave).  mcs_get_launch returns the value set */
     int32_t refill_min;        /* idle lanes that trigger a wave refill 1..64 */
     int32_t coop_live;         /* native mode, once the work queue is empty: a
                                   wave with at most this many live photons

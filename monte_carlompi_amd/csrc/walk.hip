@@ -30,6 +30,7 @@
 #include <mutex>
 #include <new>
 #include <thread>
+#include <type_traits>
 #include <vector>
 
 #include "mcsnow.h"
@@ -528,6 +529,144 @@ __device__ void hg_tail(NativeWalker &w, int &state, const KParams &P, int wave)
     }
 }
 
+// Tail mode of the replay walk (no phase matrices).  A step of it is ~450 FP64
+// instructions, most of them independent of the photon's state: the logarithm,
+// sine, cosine, the scattering cosine's division and root, the path's division.
+// Once the queue is empty and a wave holds at most RP_TAIL photons, the lanes of
+// a photon's group build those of its next G = 64 / 2^ceil(log2 L) steps from
+// its five deviates each, and its own lane then only rotates and moves, up to
+// the first step in which a photon of the wave exits, is absorbed, runs out of
+// deviates or reaches the step cap.  Steps of another kind (the first, the one
+// after a bottom reflection, the surface mode, the last deviates of a slice)
+// are taken by step().  The expressions and their order are step()'s, so the
+// records are the same bit for bit.  LDS: one RpTab per wave.  A lone photon's
+// step takes 0.35 us instead of 2.1 (rotation: a root and two divisions in
+// FP64); 20,000 photons, longest walk 706 steps: kernel 1.72 -> 0.32 ms at the
+// (256, 4, 512) shape, with the photons dealt over the chip (walk_shape).
+constexpr int RP_TAIL = 32;
+struct RpTab {
+    double dtau[64], path[64], cost[64], sint[64], cosp[64], sinp[64];
+    int own[RP_TAIL];
+};
+__device__ __forceinline__ double bperm(int src_lane, double v)
+{
+    const uint64_t b = (uint64_t)__double_as_longlong(v);
+    const uint32_t lo = bperm(src_lane, (uint32_t)b), hi = bperm(src_lane, (uint32_t)(b >> 32));
+    return __longlong_as_double((long long)(((uint64_t)hi << 32) | lo));
+}
+__device__ __forceinline__ int64_t bperm(int src_lane, int64_t v)
+{
+    return (int64_t)(((uint64_t)bperm(src_lane, (uint32_t)((uint64_t)v >> 32)) << 32) | bperm(src_lane, (uint32_t)(uint64_t)v));
+}
+__device__ void rp_tail(ReplayWalker &w, int &state, const KParams &P, int wave)
+{
+#pragma clang fp contract(off)
+    extern __shared__ __align__(16) RpTab rp_tab[];
+    RpTab &tab = rp_tab[wave];
+    const int lane = lane_id();
+    unsigned long long em = 0ull;              // photons of the grouping (0: regroup)
+    int lg = 0, G = 64;
+    int64_t pos = 0, end = 0;
+    double g = 0.0, ext = 1.0, ssa_ice = 1.0, ssa_imp = 1.0, p_imp = 0.0;
+    bool member = false;
+    for (;;) {
+        if (__ballot(state == LIVE) == 0ull) break;
+        // steps of another kind
+        const auto plain = [&] { return w.i == 0u || w.bounce || w.surf || w.pos + 5 > w.end; };
+        const bool other = state == LIVE && plain();
+        if (__ballot(other)) em = 0ull;
+        if (other) {
+            const bool d = w.step(P);
+            if (d || w.i >= P.max_steps) {
+                if (!d) w.cond = 0;
+                state = DONE;
+            }
+        }
+        const bool mine = state == LIVE && !plain();
+        const unsigned long long em_now = __ballot(mine);
+        if (em_now == 0ull) continue;
+        if (em_now != em) {
+            em = em_now;
+            const int L = __popcll(em);
+            lg = (L <= 1) ? 0 : 32 - __clz(L - 1);
+            G = 64 >> lg;
+            if (mine) tab.own[lane_rank(em)] = lane;
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+            const int grp = lane >> (6 - lg);
+            member = grp < L;
+            const int o = tab.own[member ? grp : 0];
+            pos = bperm(o, w.pos);
+            end = bperm(o, w.end);
+            g = bperm(o, w.g); ext = bperm(o, w.ext_cff);
+            ssa_ice = bperm(o, w.ssa_ice); ssa_imp = bperm(o, w.ssa_imp); p_imp = bperm(o, w.p_ext_imp);
+        }
+        const int64_t at = pos + 5 * (lane & (G - 1));
+        const bool has = member && at + 5 <= end;
+        bool absorbed = false;
+        if (has) {
+            const double *d = P.rdev + at;
+            const double d0 = d[0], d1 = d[1], d2 = d[2], d3 = d[3], d4 = d[4];
+            double cost, sint;
+            ReplayWalker::polar_angle(g, d0, cost, sint);
+            const double ph = d1 * (2.0 * PI_D);
+            const double dtau = -log(d2);
+            tab.dtau[lane] = dtau;
+            tab.path[lane] = dtau / ext;
+            tab.cost[lane] = cost; tab.sint[lane] = sint;
+            tab.cosp[lane] = cos(ph); tab.sinp[lane] = sin(ph);
+            absorbed = d3 >= (d4 > p_imp ? ssa_ice : ssa_imp);
+        }
+        // steps of this round, for all photons of the wave: through the first
+        // absorption, before the first that lacks deviates
+        unsigned long long am = __ballot(absorbed), nm = __ballot(member && !has);
+        for (int h = 32; h >= G; h >>= 1) {
+            am |= am >> h;
+            nm |= nm >> h;
+        }
+        const unsigned long long low = G == 64 ? ~0ull : (1ull << G) - 1ull;
+        am &= low;
+        nm &= low;
+        int ns = am ? __ffsll((long long)am) : G;
+        if (nm) ns = min(ns, __ffsll((long long)nm) - 1);   // >= 1: every photon has five
+        if (__ballot(mine && P.max_steps - w.i < (uint32_t)G)) ns = 1;
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        int k = 0;
+        bool ended = false;
+        if (mine) {
+            const int b = lane_rank(em) * G;
+            double z_prev = w.z, dtau = 0.0;
+            do {
+                double x, y, u;
+                w.rotate(tab.cost[b + k], tab.sint[b + k], tab.cosp[b + k], tab.sinp[b + k], x, y, u);
+                dtau = tab.dtau[b + k];
+                z_prev = w.z;
+                w.z = z_prev + dtau * u;
+                w.mux = x; w.muy = y; w.muz = u;
+                w.muz2 = u * u;
+                w.path += tab.path[b + k];
+                ++k;
+            } while (__ballot(w.z > 0.0 || w.z < -w.tau_tot) == 0ull && k < ns);
+            w.i += (uint32_t)k;
+            w.pos += 5 * k;
+            w.u_ssa = P.rdev[w.pos - 2];
+            w.u_ext = P.rdev[w.pos - 1];
+            const bool ev = w.z > 0.0 || w.z < -w.tau_tot || w.u_ssa >= (w.u_ext > w.p_ext_imp ? w.ssa_ice : w.ssa_imp);
+            bool d = false;
+            if (ev) {
+                d = w.event(P, dtau, z_prev);
+                ended = true;
+            }
+            if (d || w.i >= P.max_steps) {
+                if (!d) w.cond = 0;
+                state = DONE;
+            }
+        }
+        if (__ballot(ended)) em = 0ull;        // a reflection drew a deviate: regroup
+        else pos += 5 * __builtin_amdgcn_readlane(k, __ffsll((long long)em) - 1);
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    }
+}
+
 // Wave issue priority from the oldest live photon (i = its step count, 0 for
 // other lanes): long walks set the tail of a launch, so their waves win issue
 // slots over young ones.
@@ -644,8 +783,17 @@ k_walk(const KParams P)
                 break;
             }
         }
+        constexpr bool RTAIL = std::is_same<W, ReplayWalker>::value;
+        if constexpr (RTAIL) {
+            // queue empty and few photons left: the replay tail
+            if (lds_load(&bs.exhausted) && __popcll(live) <= RP_TAIL) {
+                rp_tail(w, state, P, wave);
+                retire<W, DIRECT>(bs, P, w, state, my_slot, my_gid);
+                break;
+            }
+        }
         constexpr bool PTAIL = W::STOKES && !W::COOP && sizeof(typename W::Real) == 4;
-        const int ptail = PTAIL ? min(P.coop_live, 16) : 0;
+        const int ptail = RTAIL ? RP_TAIL : PTAIL ? min(P.coop_live, 16) : 0;
         if constexpr (PTAIL) {
             // polarised walk: queue empty, few photons, all with the exact sampler
             if (ptail > 0 && lds_load(&bs.exhausted) && __popcll(live) <= ptail &&
@@ -1521,12 +1669,14 @@ static int64_t count_chunks(const mcs_ctx *c, int chunk)
 //   records do not depend on the shape (coop_live 0, polarised, replay) then
 //   shrink their chunks to one per block (500,000 photons at the default
 //   shape, coop_live 0: kernel 2.00 -> 1.86 ms; polarised 300,000: 1.89 -> 1.32).
-// * Native walks that have a lane for every photon take the ONE form of k_walk:
+// * Walks that have a lane for every photon (replays without phase matrices,
+//   native walks) take the ONE form of k_walk:
 //   as many blocks as are resident together, the photons spread evenly over
 //   them.  Kernel ms at the default shape (256, 4, 2048, 8), queue -> ONE:
 //   coop_live 0: 2,000 photons 1.50 -> 0.70, 10,000 1.53 -> 0.76, 250,000 1.98
 //   -> 1.54 (0.36, 0.41 and 1.05 since hg_tail runs in batches); polarised: 2,000 1.51 -> 0.43, 20,000 1.82 -> 0.77, 100,000 1.96 ->
-//   1.02.  Polarised blocks of 512 threads, one per CU, hold the photons up to
+//   1.02; replay, whose tail holds up to 32 photons a wave: 2,000 2.2 -> 0.24,
+//   60,000 2.9 -> 0.50.  Polarised blocks of 512 threads, one per CU, hold the photons up to
 //   8 waves per CU (20,000 photons: 0.77 ms; 256-thread blocks, three per CU,
 //   0.95: three waves share a SIMD from the start, and not evenly), then
 //   256-thread blocks up to 12.  In the cooperative mode the form is taken when
@@ -1545,8 +1695,8 @@ static WalkShape walk_shape(const mcs_ctx *c, int mode)
         per_cu *= s.block / PolarWalker::MAX_BLOCK;   // same threads per CU in smaller blocks
         s.block = PolarWalker::MAX_BLOCK;
     }
-    if (!replay && n > 0) {
-        int block = s.block, blocks = std::min(per_cu, 16 / (s.block / 64));
+    if (!(replay && c->polar) && n > 0) {
+        int block = s.block, blocks = std::min(per_cu, (replay ? 4 * ReplayWalker::WAVES_PER_EU : 16) / (s.block / 64));
         if (polar) {
             const bool eight = n <= (int64_t)512 * c->cus;
             block = eight ? 512 : 256;
@@ -1556,7 +1706,7 @@ static WalkShape walk_shape(const mcs_ctx *c, int mode)
         const int64_t ch = (n + g - 1) / g;
         const int waves = block / 64;
         const int64_t take = (ch + waves - 1) / waves;
-        if (ch <= block && (polar || coop == 0 || take <= coop)) {
+        if (ch <= block && (replay || polar || coop == 0 || take <= coop)) {
             const int64_t nch = count_chunks(c, (int)ch);
             if (nch <= g) {
                 s.block = block;
@@ -1650,9 +1800,16 @@ static int enqueue_walk(mcs_ctx *c, int mode, const KParams &P, const WalkShape 
             direct ? go(k_walk<NativeWalker, 5, true>) : go(k_walk<NativeWalker, 5>);
         else
             direct ? go(k_walk<NativeWalker, 6, true>) : go(k_walk<NativeWalker, 6>);
+    } else if (c->polar) {
+        using W = ReplayWalkerT<true>;
+        hipLaunchKernelGGL((k_walk<W, W::WAVES_PER_EU>), dim3(grid), dim3(block), 0, c->stream, P);
     } else {
-        hipLaunchKernelGGL((k_walk<ReplayWalker, ReplayWalker::WAVES_PER_EU>), dim3(grid), dim3(block), 0,
-                           c->stream, P);
+        using W = ReplayWalker;
+        const size_t tab = (size_t)(block / 64) * sizeof(RpTab);
+        if (shape.take > 0)
+            hipLaunchKernelGGL((k_walk<W, W::WAVES_PER_EU, false, 1, true>), dim3(grid), dim3(block), tab, c->stream, P);
+        else
+            hipLaunchKernelGGL((k_walk<W, W::WAVES_PER_EU>), dim3(grid), dim3(block), tab, c->stream, P);
     }
     if (events && hipEventRecord(c->ev1, c->stream) != hipSuccess)
         return set_err(c, MCS_ERR_HIP, "hipEventRecord failed");

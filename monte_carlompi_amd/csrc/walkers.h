@@ -936,11 +936,13 @@ using PolarWalker = NativeWalkerT<true>;
 
 // ----------------------------------------------------------- replay walker
 // FP64, the reference's operation order; contraction off so that every
-// product and sum rounds as numpy's float64 scalars do.
-struct ReplayWalker {
+// product and sum rounds as numpy's float64 scalars do.  PM: built for
+// aspherical cases too (their code takes the 256 VGPRs and spills).
+template <bool PM>
+struct ReplayWalkerT {
     using Real = double;
     static constexpr bool COOP = false;
-    static constexpr bool STOKES = true;
+    static constexpr bool STOKES = PM;
     static constexpr bool CAP_IN_STEP = false;
     static constexpr int MAX_BLOCK = 256;
     static constexpr int WAVES_PER_EU = 2;
@@ -956,6 +958,8 @@ struct ReplayWalker {
     double sI, sQ, sU, sV;
     int pm;
     int case_id;
+
+    __device__ bool matrix() const { return PM && pm >= 0; }
 
     __device__ double draw(const KParams &P)
     {
@@ -981,7 +985,7 @@ struct ReplayWalker {
         end = P.roff[gid + 1];
         err = false;
         this->case_id = case_id;
-        pm = C.polar ? B.pm : -1;
+        pm = PM && C.polar ? B.pm : -1;
         sI = C.s0[0]; sQ = C.s0[1]; sU = C.s0[2]; sV = C.s0[3];
         dtau0 = -log(draw(P));
         u_ssa = draw(P);
@@ -995,13 +999,78 @@ struct ReplayWalker {
         return false;
     }
 
+    // cos and sin of the scattering angle from its deviate (g != 0 in the caller's case or not)
+    __device__ __forceinline__ static void polar_angle(double g, double u, double &cost, double &sint)
+    {
+#pragma clang fp contract(off)
+        if (g == 0.0) {
+            cost = 1.0 - 2.0 * u;
+        } else {
+            const double t = (1.0 - g * g) / ((1.0 - g) + (2.0 * g) * u);
+            cost = (1.0 / (2.0 * g)) * ((1.0 + g * g) - t * t);
+        }
+        sint = sqrt(1.0 - cost * cost);
+    }
+
+    // the direction after a scattering (mc3D:1255-1281)
+    __device__ __forceinline__ void rotate(double cost, double sint, double cosp, double sinp, double &mxn, double &myn,
+                                           double &mzn) const
+    {
+#pragma clang fp contract(off)
+        if (muz == 1.0) {
+            mxn = sint * cosp; myn = sint * sinp; mzn = cost;
+        } else if (muz == -1.0) {
+            mxn = sint * cosp; myn = -sint * sinp; mzn = -cost;
+        } else {
+            const double sq = sqrt(1.0 - muz2);
+            mxn = (sint * (mux * muz * cosp - muy * sinp)) / sq + mux * cost;
+            myn = (sint * (muy * muz * cosp + mux * sinp)) / sq + muy * cost;
+            mzn = -sq * sint * cosp + muz * cost;
+        }
+    }
+
+    // What follows a move of dtau from depth z_prev (z and the direction hold
+    // the state after it, path includes it): exits, the bottom's reflection,
+    // absorption by the step's u_ssa and u_ext; true when the walk has ended
+    __device__ __forceinline__ bool event(const KParams &P, double dtau, double z_prev)
+    {
+#pragma clang fp contract(off)
+        const double z_i = z;
+        const bool ice = u_ext > p_ext_imp;
+        const double ssa_event = surf ? R : (ice ? ssa_ice : ssa_imp);   // mc3D:1374-1387
+        if (z_i > 0.0) {
+            path += -((z_i * dtau) / ((z_i - z_prev) * ext_cff));
+            cond = 1;
+            return true;
+        }
+        if (z_i < -tau_tot) {
+            path += -(((z_i + tau_tot) * dtau) / ((z_i - z_prev) * ext_cff));
+            const double dcorr = -(((z_i + tau_tot) / (z_prev - z_i)) * dtau);
+            z = z_i - (muz * dcorr);
+            const int exit_cond = (i == 1) ? 3 : 2;
+            if (lamb) {
+                if (draw(P) <= R) {
+                    bounce = true;
+                    return err;
+                }
+            }
+            cond = exit_cond;
+            return true;
+        }
+        if (u_ssa >= ssa_event) {
+            cond = ice ? 4 : 5;
+            return true;
+        }
+        return err;
+    }
+
     __device__ bool step(const KParams &P)
     {
 #pragma clang fp contract(off)
         ++i;
         double dtau, u_hg = 0.0, u_phi = 0.0, p_cos = 0.0, two_phi = 0.0;
         if (i >= 2) {
-            if (pm < 0 && pos + 5 <= end) {
+            if (!matrix() && pos + 5 <= end) {
                 // the step's five deviates are consecutive: five independent
                 // loads in flight at once instead of five dependent draws
                 const double *d = P.rdev + pos;
@@ -1013,7 +1082,7 @@ struct ReplayWalker {
                 u_ssa = d3;
                 u_ext = d4;
             } else {
-                if (pm >= 0) {
+                if (matrix()) {
                     polar_draws(P, p_cos, two_phi);
                 } else {
                     u_hg = draw(P);
@@ -1041,70 +1110,30 @@ struct ReplayWalker {
                         break;
                     }
                 }
-            } else if (pm >= 0) {
+            } else if (matrix()) {
                 cost = p_cos;
                 sint = sqrt(1.0 - cost * cost);
-            } else if (g == 0.0) {
-                cost = 1.0 - 2.0 * u_hg;
-                sint = sqrt(1.0 - cost * cost);
             } else {
-                const double t = (1.0 - g * g) / ((1.0 - g) + (2.0 * g) * u_hg);
-                cost = (1.0 / (2.0 * g)) * ((1.0 + g * g) - t * t);
-                sint = sqrt(1.0 - cost * cost);
+                polar_angle(g, u_hg, cost, sint);
             }
-            const double ph = (pm >= 0) ? two_phi / 2.0 : u_phi * (2.0 * PI_D);
+            const double ph = matrix() ? two_phi / 2.0 : u_phi * (2.0 * PI_D);
             const double cosp = cos(ph), sinp = sin(ph);
-            if (muz == 1.0) {
-                mxn = sint * cosp; myn = sint * sinp; mzn = cost;
-            } else if (muz == -1.0) {
-                mxn = sint * cosp; myn = -sint * sinp; mzn = -cost;
-            } else {
-                const double sq = sqrt(1.0 - muz2);
-                mxn = (sint * (mux * muz * cosp - muy * sinp)) / sq + mux * cost;
-                myn = (sint * (muy * muz * cosp + mux * sinp)) / sq + muy * cost;
-                mzn = -sq * sint * cosp + muz * cost;
-            }
+            rotate(cost, sint, cosp, sinp, mxn, myn, mzn);
             if (bounce) {                        // mc3D:1283-1285
                 sI = 1.0; sQ = 0.0; sU = 0.0; sV = 0.0;
-            } else if (pm >= 0) {                // mc3D:1287-1342
+            } else if (matrix()) {               // mc3D:1287-1342
                 stokes_update(P, cost, cosp, mzn, muz);
             }
             bounce = false;
         }
         const double z_prev = z;
-        const double z_i = z_prev + dtau * mzn;
-        z = z_i;
+        z = z_prev + dtau * mzn;
         if (i > 1) {
             mux = mxn; muy = myn; muz = mzn;
             muz2 = muz * muz;
         }
         path += dtau / ext_cff;
-        const bool ice = u_ext > p_ext_imp;
-        const double ssa_event = surf ? R : (ice ? ssa_ice : ssa_imp);   // mc3D:1374-1387
-        if (z_i > 0.0) {
-            path += -((z_i * dtau) / ((z_i - z_prev) * ext_cff));
-            cond = 1;
-            return true;
-        }
-        if (z_i < -tau_tot) {
-            path += -(((z_i + tau_tot) * dtau) / ((z_i - z_prev) * ext_cff));
-            const double dcorr = -(((z_i + tau_tot) / (z_prev - z_i)) * dtau);
-            z = z_i - (mzn * dcorr);
-            const int exit_cond = (i == 1) ? 3 : 2;
-            if (lamb) {
-                if (draw(P) <= R) {
-                    bounce = true;
-                    return err;
-                }
-            }
-            cond = exit_cond;
-            return true;
-        }
-        if (u_ssa >= ssa_event) {
-            cond = ice ? 4 : 5;
-            return true;
-        }
-        return err;
+        return event(P, dtau, z_prev);
     }
 
     // populate_pdfs for an aspherical particle (mc3D:898-1004): area, cos
@@ -1223,6 +1252,7 @@ struct ReplayWalker {
         else { phi = __builtin_nan(""); axis = true; }
     }
 };
+using ReplayWalker = ReplayWalkerT<false>;
 
 
 // Lanes are EMPTY (no photon), LIVE or DONE (finished, record pending).

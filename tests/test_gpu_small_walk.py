@@ -1,5 +1,5 @@
-"""Native walks whose photons fit in the launch's lanes run one chunk per block
-(no queue); larger ones the chunk queue, replays chunks shrunk to one per block.  Both give the records of every photon
+"""Walks whose photons fit in the launch's lanes run one chunk per block (no
+queue); larger ones the chunk queue.  Both give the records of every photon
 bit for bit (coop_live 0, polarised and replay walks), at the sizes around the
 line between them, for one and for several cases, into the context's buffers
 and into a caller's."""
@@ -72,11 +72,16 @@ def test_polar(walker, tmp_path, n):
         assert_same(records(walker, shape, [case], stokes=True), ref, FIELDS + ('Q_n', 'U_n', 'V_n'))
 
 
-def test_replay_chunks(walker):
-    golden = [c for c in load()[1] if c['name'] == 'thin_lamb'][0]
+@pytest.mark.parametrize('name', [c['name'] for c in load()[1] if not c['lowprec_columns']])
+def test_replay_chunks(walker, name):
+    """The queue and the ONE form, with the tail that builds a photon's next
+    steps in the idle lanes, on the reference's own streams (Lambertian bottoms
+    and surfaces among them)."""
+    golden = [c for c in load()[1] if c['name'] == name][0]
     _, par, values, offsets = run_case(golden)
     k = 64 * walker.cus // golden['n'] + 2                 # past the queue shape's lanes
-    case, band = case_from_params(par, golden['tau'], META['rho_snw'], golden['theta0'], golden['lb'], golden['R'])
+    case, band = case_from_params(par, golden['tau'], META['rho_snw'], golden['theta0'], golden['lb'], golden['R'],
+                                  golden.get('ls', False))
     case.n_photons = k * golden['n']
     off = np.concatenate([[0], (offsets[-1] * np.arange(k)[:, None] + offsets[1:][None, :]).ravel()])
     kw = dict(mode='replay', replay=(np.tile(values, k), off), photon_band=np.tile(band, k))
