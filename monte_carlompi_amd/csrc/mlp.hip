@@ -22,6 +22,7 @@
 #include <vector>
 
 #include "mcsnow.h"
+#include "host_copy.h"
 
 namespace mlp {
 
@@ -463,6 +464,7 @@ struct mcs_mlp {
     float *xd = nullptr, *td = nullptr;
     int64_t n_data = 0;
     double last_ms = 0.0;
+    HostCopy copier;                 // large copies to pageable host arrays
     // serving (mcs_mlp_set_serving): input feature map, its standardisation
     // (K0 floats each) and the output transform (n_out floats each)
     int32_t feature_map = MCS_FEATURES_IDENTITY;
@@ -852,6 +854,7 @@ int mcs_mlp_destroy(mcs_mlp *c)
     if (!c) return MCS_ERR_ARG;
     (void)hipSetDevice(c->device);
     if (c->stream) (void)hipStreamSynchronize(c->stream);
+    c->copier.release();
     void *bufs[] = {c->p, c->gr, c->m, c->v, c->mask, c->pb_index, c->wb, c->X, c->dY, c->dZa, c->dZb,
                     c->Y, c->T, c->w, c->yout, c->xin, c->loss, c->idx, c->xd, c->td,
                     c->fmu, c->fsd, c->oscale, c->oshift, c->ooff, c->lpart, c->ws, c->wf, c->wt, c->part, c->didx};
@@ -943,8 +946,7 @@ int mcs_mlp_forward(mcs_mlp *c, const float *x, int64_t n, float *y)
         }
         MCHK(c, hipEventRecord(c->e1, c->stream));
         MCHK(c, hipGetLastError());
-        MCHK(c, hipMemcpyAsync(y + s * no, c->yout, sizeof(float) * rows * no, hipMemcpyDeviceToHost, c->stream));
-        MCHK(c, hipStreamSynchronize(c->stream));
+        MCHK(c, c->copier.run((char *)(y + s * no), (char *)c->yout, sizeof(float) * rows * no, true, c->stream));
         float ms = 0.f;
         MCHK(c, hipEventElapsedTime(&ms, c->e0, c->e1));
         total_ms += ms;

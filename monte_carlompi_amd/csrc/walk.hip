@@ -34,6 +34,7 @@
 #include <vector>
 
 #include "mcsnow.h"
+#include "host_copy.h"
 #include "philox.h"
 #include "walk_state.h"
 #include "walkers.h"
@@ -1110,6 +1111,7 @@ struct mcs_ctx {
     // pinned host staging of record read-back (grown on demand)
     void *h_stage = nullptr;
     size_t stage_cap = 0;
+    HostCopy copier;                 // uploads of recorded streams from pageable arrays
     // device address of the mcs_walk_noalloc scratch on this context's device
     unsigned long long *noalloc_scratch = nullptr;
     hipError_t noalloc_err = hipSuccess;
@@ -1277,26 +1279,6 @@ static void parallel_rows(int64_t n, F f)
     for (auto &x : th) x.join();
 }
 
-// [p, p + bytes) lies in one pinned (page-locked, hipHostMalloc) host
-// allocation: the DMA engine can write it directly.
-static bool host_pinned(const void *p, size_t bytes)
-{
-    hipPointerAttribute_t a;
-    if (hipPointerGetAttributes(&a, p) != hipSuccess) {
-        (void)hipGetLastError();   // pageable memory: the query reports invalid value
-        return false;
-    }
-    if (a.type != hipMemoryTypeHost) return false;
-    void *start = nullptr;
-    size_t size = 0;
-    if (hipPointerGetAttribute(&start, HIP_POINTER_ATTRIBUTE_RANGE_START_ADDR, (hipDeviceptr_t)p) != hipSuccess ||
-        hipPointerGetAttribute(&size, HIP_POINTER_ATTRIBUTE_RANGE_SIZE, (hipDeviceptr_t)p) != hipSuccess) {
-        (void)hipGetLastError();
-        return false;
-    }
-    return (const char *)p >= (const char *)start && (const char *)p + bytes <= (const char *)start + size;
-}
-
 // Copy k device columns (d_wide + off[k], n * esz[k] bytes) to the host
 // arrays dst[k] (nullable): pinned destinations by one DMA each, the others
 // into pinned staging and from there by host threads.  Waits for the stream.
@@ -1378,6 +1360,7 @@ int mcs_destroy(mcs_ctx *c)
     if (c->ev1) (void)hipEventDestroy(c->ev1);
     if (c->h_sum) (void)hipHostFree(c->h_sum);
     if (c->h_stage) (void)hipHostFree(c->h_stage);
+    c->copier.release();
     if (c->stream) (void)hipStreamDestroy(c->stream);
     delete c;
     return MCS_OK;
@@ -1920,7 +1903,8 @@ int mcs_walk(mcs_ctx *c, const mcs_walk_args *a)
     if (a->mode == MCS_REPLAY) {
         if ((r = ensure(c, c->d_rdev, sizeof(double) * (size_t)rlen))) return r;
         if ((r = ensure(c, c->d_roff, sizeof(int64_t) * (size_t)(n + 1)))) return r;
-        HIPCHK(c, hipMemcpyAsync(c->d_rdev.p, a->replay_dev, sizeof(double) * (size_t)rlen, hipMemcpyHostToDevice, c->stream));
+        HIPCHK(c, c->copier.run((char *)const_cast<double *>(a->replay_dev), (char *)c->d_rdev.p,
+                                sizeof(double) * (size_t)rlen, false, c->stream));
         HIPCHK(c, hipMemcpyAsync(c->d_roff.p, a->replay_off, sizeof(int64_t) * (size_t)(n + 1), hipMemcpyHostToDevice, c->stream));
     }
     const size_t rsz = (a->mode == MCS_NATIVE) ? 4 : 8;
