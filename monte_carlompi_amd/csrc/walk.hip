@@ -542,7 +542,7 @@ __device__ void hg_tail(NativeWalker &w, int &state, const KParams &P, int wave)
 // are taken by step().  The expressions and their order are step()'s, so the
 // records are the same bit for bit.  LDS: one RpTab per wave.  A lone photon's
 // step takes 0.35 us instead of 2.1 (rotation: a root and two divisions in
-// FP64); 20,000 photons, longest walk 706 steps: kernel 1.72 -> 0.32 ms at the
+// FP64); 20,000 photons, longest walk 706 steps: kernel 1.68 -> 0.33 ms at the
 // (256, 4, 512) shape, with the photons dealt over the chip (walk_shape).
 constexpr int RP_TAIL = 32;
 struct RpTab {
@@ -1653,19 +1653,20 @@ static int64_t count_chunks(const mcs_ctx *c, int chunk)
 //   shrink their chunks to one per block (500,000 photons at the default
 //   shape, coop_live 0: kernel 2.00 -> 1.86 ms; polarised 300,000: 1.89 -> 1.32).
 // * Walks that have a lane for every photon (replays without phase matrices,
-//   native walks) take the ONE form of k_walk:
-//   as many blocks as are resident together, the photons spread evenly over
-//   them.  Kernel ms at the default shape (256, 4, 2048, 8), queue -> ONE:
-//   coop_live 0: 2,000 photons 1.50 -> 0.70, 10,000 1.53 -> 0.76, 250,000 1.98
-//   -> 1.54 (0.36, 0.41 and 1.05 since hg_tail runs in batches); polarised: 2,000 1.51 -> 0.43, 20,000 1.82 -> 0.77, 100,000 1.96 ->
-//   1.02; replay, whose tail holds up to 32 photons a wave: 2,000 2.2 -> 0.24,
-//   60,000 2.9 -> 0.50.  Polarised blocks of 512 threads, one per CU, hold the photons up to
-//   8 waves per CU (20,000 photons: 0.77 ms; 256-thread blocks, three per CU,
-//   0.95: three waves share a SIMD from the start, and not evenly), then
-//   256-thread blocks up to 12.  In the cooperative mode the form is taken when
-//   its waves hold at most coop_live photons each, so that they start in the
-//   tail (10,000 photons 0.90 -> 0.08 ms, 50,000 0.94 -> 0.12); above that the
-//   caller's shape says how many photons finish cooperatively.
+//   native walks) take the ONE form of k_walk: as many blocks as are resident
+//   together, the photons spread evenly over them.  Kernel ms at the default
+//   shape (256, 4, 2048, 8), queue -> ONE: coop_live 0: 2,000 photons 1.50 ->
+//   0.70, 10,000 1.53 -> 0.76, 250,000 1.98 -> 1.54 (0.36, 0.41 and 1.05 since
+//   hg_tail runs in batches); polarised: 2,000 1.51 -> 0.43, 20,000 1.82 ->
+//   0.77, 100,000 1.96 -> 1.02; replay with rp_tail, (256, 4, 512, 8): 2,000
+//   1.46 -> 0.24, 20,000 1.68 -> 0.33, 60,000 2.2 -> 0.49.  Polarised blocks of
+//   512 threads, one per CU, hold the photons up to 8 waves per CU (20,000
+//   photons: 0.77 ms; 256-thread blocks, three per CU, 0.95: three waves share
+//   a SIMD from the start, and not evenly), then 256-thread blocks up to 12.
+//   In the cooperative mode the form is taken when its waves hold at most
+//   coop_live photons each, so that they start in the tail (10,000 photons 0.90
+//   -> 0.08 ms, 50,000 0.94 -> 0.12); above that the caller's shape says how
+//   many photons finish cooperatively.
 static WalkShape walk_shape(const mcs_ctx *c, int mode)
 {
     WalkShape s;
