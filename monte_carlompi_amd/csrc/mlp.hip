@@ -268,22 +268,29 @@ __device__ __forceinline__ SnowInputs snow_inputs(const float *q)
     s.mu0 = cos((double)q[3] * (3.141592653589793 / 180.0));
     return s;
 }
-__device__ __forceinline__ float snow_feature(const SnowInputs &s, int k, const float *mu, const float *sd)
+// Standardised feature k as the network's input.  The first is rounded to BF16
+// straight from FP64, the others by way of FP32: where the FP32 value is a BF16
+// tie (7 of 1e6 random r_eff) the two differ by one BF16 step, so the
+// intermediate is kept from being folded away (the empty asm).
+__device__ __forceinline__ bf16 snow_feature(const SnowInputs &s, int k, const float *mu, const float *sd)
 {
     // the standardisation in every branch, beside the feature it may be
     // contracted with: every caller then rounds alike
     const double m = mu[k], d = sd[k];
+    float f;
     switch (k) {
-    case 0: return (float)((log(s.reff) - m) / d);
-    case 1: return (float)((log10(fmax(1.0 - s.om, 1e-12)) - m) / d);
-    case 2: return (float)((s.g - m) / d);
-    case 3: return (float)((s.mu0 - m) / d);
-    case 4: return (float)((log10(s.tau) - m) / d);
-    case 5: return (float)((exp(-s.tau / s.mu0) - m) / d);
-    case 6: return (float)((sqrt((1.0 - s.om) / (1.0 - s.om * s.g)) - m) / d);
-    case 7: return (float)((log10(s.tau * (1.0 - s.om * s.g)) - m) / d);
-    default: return (float)((log10(s.tau / s.mu0) - m) / d);
+    case 0: return (bf16)((log(s.reff) - m) / d);
+    case 1: f = (float)((log10(fmax(1.0 - s.om, 1e-12)) - m) / d); break;
+    case 2: f = (float)((s.g - m) / d); break;
+    case 3: f = (float)((s.mu0 - m) / d); break;
+    case 4: f = (float)((log10(s.tau) - m) / d); break;
+    case 5: f = (float)((exp(-s.tau / s.mu0) - m) / d); break;
+    case 6: f = (float)((sqrt((1.0 - s.om) / (1.0 - s.om * s.g)) - m) / d); break;
+    case 7: f = (float)((log10(s.tau * (1.0 - s.om * s.g)) - m) / d); break;
+    default: f = (float)((log10(s.tau / s.mu0) - m) / d); break;
     }
+    asm volatile("" : "+v"(f));
+    return (bf16)f;
 }
 __global__ void k_features_snow(const float *in, int rows, const float *mu, const float *sd, bf16 *X)
 {
@@ -292,7 +299,7 @@ __global__ void k_features_snow(const float *in, int rows, const float *mu, cons
     const SnowInputs s = snow_inputs(in + (size_t)r * 5);
     bf16 *row = X + (size_t)r * K0;
 #pragma unroll
-    for (int k = 0; k < K0; ++k) row[k] = (bf16)(k < SNOW_FEATURES ? snow_feature(s, k, mu, sd) : 0.f);
+    for (int k = 0; k < K0; ++k) row[k] = k < SNOW_FEATURES ? snow_feature(s, k, mu, sd) : (bf16)0.f;
 }
 
 // minibatch gather from the resident dataset

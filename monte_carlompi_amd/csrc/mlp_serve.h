@@ -77,7 +77,7 @@ __global__ void __launch_bounds__(SV_WAVES * 64) __attribute__((amdgpu_waves_per
         const float *q = g.x + (in ? r0 + row : 0) * 5;
         const SnowInputs s = snow_inputs(q);
         for (int k = sub; k < K0; k += SUBS)
-            Act[row * SV_PITCH_X + k] = (bf16)(k < SNOW_FEATURES && in ? snow_feature(s, k, g.fmu, g.fsd) : 0.f);
+            Act[row * SV_PITCH_X + k] = k < SNOW_FEATURES && in ? snow_feature(s, k, g.fmu, g.fsd) : (bf16)0.f;
     } else {
         for (int i = t; i < R * K0; i += SV_WAVES * 64) {
             const int row = i / K0, c = i % K0;
