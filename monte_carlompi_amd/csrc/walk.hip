@@ -425,8 +425,11 @@ struct HgTab {
 static_assert(sizeof(HgTab) % 16 == 0, "HgTab: 16-byte LDS loads");
 __device__ void hg_tail(NativeWalker &w, int &state, const KParams &P, int wave)
 {
-    extern __shared__ __align__(16) CoopEntry coop_tab[];
-    HgTab &tab = reinterpret_cast<HgTab *>(coop_tab)[wave];
+    // under a name of its own: one declaration's alignment holds for all of that
+    // name, and the cooperative tables at 16 bytes cost the 6-wave instance
+    // nine scratch reloads (its walks 3 % slower)
+    extern __shared__ HgTab hg_tabs[];
+    HgTab &tab = hg_tabs[wave];
     const int lane = lane_id();
     unsigned long long em = 0ull;              // live photons of the grouping (0: regroup)
     int lg = 0, G = 64;
