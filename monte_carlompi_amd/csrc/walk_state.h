@@ -114,10 +114,10 @@ struct KParams {
     int32_t pm_n;
     int32_t pm_lds_floats;       // > 0: the FP32 tables are copied into dynamic LDS at block start
     int32_t pm_stride;
-    uint32_t take;               // k_walk's ONE form: photons per wave (0: the queue form)
     int32_t rec_direct;          // 1: records go straight to photon order (pos = gid), no compaction
     void *rec_stokes;
     uint64_t n_total;
+    uint32_t take;               // ONE form: photons per wave, else 0 (last: the loads of the others stay as they pair)
 };
 
 // ---------------------------------------------------------------- LDS state
