@@ -504,19 +504,22 @@ static hipError_t dalloc(T **p, size_t count)
     return hipMalloc((void **)p, sizeof(T) * std::max<size_t>(count, 1));
 }
 
+// Long-K products with few output tiles (weight gradients): K in chunks, a
+// multiple of BK each, so that ~512 blocks run.  Both training paths sum the
+// batch in these chunks.
+static int split_k(int M, int N, int K)
+{
+    const int tiles = ((N + BN - 1) / BN) * ((M + BM - 1) / BM);
+    const int splits = std::max(1, std::min(K / BK, (512 + tiles - 1) / tiles));
+    return ((K + splits - 1) / splits + BK - 1) / BK * BK;
+}
+
 template <bool AT, bool BT, int EPI>
 static void gemm(mcs_mlp *c, const GemmArgs &g0)
 {
     GemmArgs g = g0;
-    const int tiles = ((g.N + BN - 1) / BN) * ((g.M + BM - 1) / BM);
-    int splits = 1;
-    if (EPI == EPI_ADD_F32) {
-        // long-K products with few output tiles (weight gradients): split K so
-        // that ~512 blocks run, slices a multiple of BK
-        splits = std::max(1, std::min(g.K / BK, (512 + tiles - 1) / tiles));
-    }
-    g.kchunk = ((g.K + splits - 1) / splits + BK - 1) / BK * BK;
-    splits = (g.K + g.kchunk - 1) / g.kchunk;
+    g.kchunk = EPI == EPI_ADD_F32 ? split_k(g.M, g.N, g.K) : (g.K + BK - 1) / BK * BK;
+    const int splits = (g.K + g.kchunk - 1) / g.kchunk;
     dim3 grid((g.N + BN - 1) / BN, (g.M + BM - 1) / BM, splits);
     hipLaunchKernelGGL((k_gemm<AT, BT, EPI>), grid, dim3(256), 0, c->stream, g);
 }
@@ -685,8 +688,8 @@ static void backward_pass(mcs_mlp *c, int rows, float *loss_out)
 }
 
 // ---- training of 256-wide networks (mlp_train.h): three kernels a step.  At
-// batch 4096 and 9 -> 4 x 256 -> 651 on MI355X k_train_rows takes 27 us,
-// k_train_dw 10 and k_train_adam 7 (the per-layer kernels, which other widths,
+// batch 4096 and 9 -> 4 x 256 -> 651 on MI355X k_train_rows takes 28 us,
+// k_train_dw 12 and k_train_adam 7 (the per-layer kernels, which other widths,
 // deeper or wider-output networks use: 26 launches, 234 us); 48 steps with
 // their uploads 11.2 -> 2.45 ms.
 static void pack_weights(mcs_mlp *c)
@@ -695,10 +698,21 @@ static void pack_weights(mcs_mlp *c)
                        c->wb, c->wf, c->wt);
 }
 
-// Partial gradients (c->part, `slices` of them) and per-block loss sums
-// (c->lpart, batch / TR_ROWS) of `batch` rows: idx into x, t (n_data rows), or
-// the first `batch` rows (idx null).
-static int rows_backward(mcs_mlp *c, const float *x, const float *t, int64_t n_data, const int32_t *idx, int batch)
+// Slices of the batch (whole chunks) for a layer's weight gradients: of eight
+// 64-row stages each, or as many as make eight slices where that is less (small
+// batches would leave the chip idle), at most DW_SLICES.
+static int dw_slices(int batch, int kc, int chunks)
+{
+    const int stages = (kc + 63) / 64, want = std::min(8, batch / 64);
+    int per = std::max(1, std::min(8 / stages, (chunks + want - 1) / want));
+    per = std::max(per, (chunks + DW_SLICES - 1) / DW_SLICES);
+    return (chunks + per - 1) / per;
+}
+
+// Partial gradients (c->part) and per-block loss sums (c->lpart, batch /
+// TR_ROWS) of `batch` rows: idx into x, t (n_data rows), or the first `batch`
+// rows (idx null).
+static GradParts rows_backward(mcs_mlp *c, const float *x, const float *t, int64_t n_data, const int32_t *idx, int batch)
 {
     const int L = c->d.n_hidden_layers;
     TrainArgs g;
@@ -710,11 +724,11 @@ static int rows_backward(mcs_mlp *c, const float *x, const float *t, int64_t n_d
     g.ld = batch + LD_PAD;
     g.p = c->p; g.w = c->w; g.wf = c->wf; g.wt = c->wt;
     g.xt = c->X; g.dyt = c->dY; g.lpart = c->lpart;
-    // batch slices of the weight gradients: 8, each a multiple of 64 rows
     d.L = L; d.batch = batch; d.ld = g.ld; d.n_pad = c->n_pad; d.part = c->part;
-    d.kchunk = ((batch + DW_SLICES - 1) / DW_SLICES + 63) / 64 * 64;
-    const int slices = d.slices = (batch + d.kchunk - 1) / d.kchunk;
-    int tiles = 0;
+    GradParts parts;
+    memset(&parts, 0, sizeof parts);
+    parts.part = c->part;
+    int blocks = 0;
     for (int l = 0; l <= L; ++l) {
         const Layer &ly = c->layers[l];
         g.woff[l] = ly.wb_off; g.boff[l] = ly.b_off;
@@ -722,14 +736,17 @@ static int rows_backward(mcs_mlp *c, const float *x, const float *t, int64_t n_d
             g.at[l] = c->A[l];
             g.dzt[l] = reinterpret_cast<bf16 *>(c->Z[l]);
         }
-        d.tile0[l] = tiles;
+        d.block0[l] = blocks;
+        d.kc[l] = split_k(ly.prow, ly.pcol, batch);
+        d.chunks[l] = (batch + d.kc[l] - 1) / d.kc[l];
+        parts.slices[l] = d.slices[l] = dw_slices(batch, d.kc[l], d.chunks[l]);
         d.mtiles[l] = ly.prow / 64; d.cols[l] = ly.pcol;
         d.dz[l] = l < L ? g.dzt[l] : g.dyt;
         d.in[l] = l ? g.at[l - 1] : g.xt;
         d.woff[l] = ly.w_off; d.boff[l] = ly.b_off;
-        tiles += d.mtiles[l] * ((ly.pcol + 63) / 64);
+        blocks += d.mtiles[l] * ((ly.pcol + 63) / 64) * d.slices[l];
     }
-    d.tile0[L + 1] = tiles;
+    d.block0[L + 1] = blocks;
     const auto go = [&](auto kernel) {
         hipLaunchKernelGGL(kernel, dim3(batch / TR_ROWS), dim3(TR_WAVES * 64), 0, c->stream, g);
     };
@@ -743,8 +760,8 @@ static int rows_backward(mcs_mlp *c, const float *x, const float *t, int64_t n_d
     case 7: go(k_train_rows<7>); break;
     default: go(k_train_rows<8>); break;
     }
-    hipLaunchKernelGGL(k_train_dw, dim3(tiles * slices), dim3(256), 0, c->stream, d);
-    return slices;
+    hipLaunchKernelGGL(k_train_dw, dim3(blocks), dim3(256), 0, c->stream, d);
+    return parts;
 }
 
 static int check_dims(const mcs_mlp_dims *d)
@@ -1082,9 +1099,9 @@ int mcs_mlp_grads(mcs_mlp *c, const float *x, const float *t, const float *w, in
     if (c->train_rows) {
         MCHK(c, hipMemcpy(c->xin, x, sizeof(float) * n * ni, hipMemcpyHostToDevice));
         MCHK(c, hipMemcpy(c->T, t, sizeof(float) * n * no, hipMemcpyHostToDevice));
-        const int slices = rows_backward(c, c->xin, c->T, n, nullptr, n);
+        const GradParts parts = rows_backward(c, c->xin, c->T, n, nullptr, n);
         hipLaunchKernelGGL(k_train_reduce, dim3((unsigned)((c->n_pad + 255) / 256)), dim3(256), 0, c->stream, c->pm,
-                           c->part, slices, c->gr, c->lpart, n / TR_ROWS, n, c->loss);
+                           parts, c->gr, c->lpart, n / TR_ROWS, n, c->loss);
         return finish_grads(c, grads, loss);
     }
     std::vector<float> tp((size_t)n * c->np, 0.f);
@@ -1139,7 +1156,6 @@ int mcs_mlp_train_steps(mcs_mlp *c, const int32_t *idx, int32_t n_steps, int32_t
     int adam_blocks = 0;
     if (c->train_rows) {
         adam.m = c->pm;
-        adam.part = c->part;
         adam.p = c->p; adam.mo = c->m; adam.vo = c->v;
         adam.b1 = a->beta1; adam.b2 = a->beta2; adam.eps = a->eps; adam.wd_lr = a->lr * a->weight_decay;
         adam.wf = c->wf; adam.wt = c->wt;
@@ -1161,8 +1177,7 @@ int mcs_mlp_train_steps(mcs_mlp *c, const int32_t *idx, int32_t n_steps, int32_t
         const int t = a->step + s + 1;
         const float lr_t = a->lr * std::sqrt(1.f - std::pow(a->beta2, (float)t)) / (1.f - std::pow(a->beta1, (float)t));
         if (c->train_rows) {
-            const int slices = rows_backward(c, c->xd, c->td, c->n_data, rows, batch);
-            adam.slices = slices;
+            adam.g = rows_backward(c, c->xd, c->td, c->n_data, rows, batch);
             adam.lr_t = lr_t;
             adam.loss = loss_out;
             hipLaunchKernelGGL(k_train_adam, dim3(adam_blocks), dim3(256), 0, c->stream, adam);

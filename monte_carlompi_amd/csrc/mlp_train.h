@@ -263,19 +263,24 @@ __global__ void __launch_bounds__(TR_WAVES * 64) __attribute__((amdgpu_waves_per
 
 // Weight and bias gradients of every layer: dW_l = dZ_l^T A_{l-1} summed over
 // the batch, both operands [feature][row] (k_train_rows), so tiles load along
-// the batch.  64 x 64 tiles of all layers in one launch (96 for the surrogate),
-// the batch in slices of `kchunk` rows: FP32 partial sums, one array of the
-// padded parameter layout per slice, added in slice order by k_train_adam /
-// k_train_reduce (no atomics, no zeroing; the same result every time).  The
-// slice runs fastest over the blocks, so with eight slices every XCD's L2 reads
-// one slice (2.8 of the surrogate's 22 MB) instead of all, the one whose rows
-// k_train_rows wrote there.  K is staged 64 rows at a time through two LDS buffers.  The tiles of
+// the batch.  64 x 64 tiles of all layers in one launch (96 for the surrogate).
+// The addends of a weight's sum are those of the per-layer kernels: chunks of
+// kc rows (split_k, another for each layer; the surrogate's at batch 4096: 32,
+// 128, 352), each one chain of MFMAs from zero.  A block adds the chunks of its
+// slice of the batch (dw_slices), one array of the padded parameter layout per
+// slice; k_train_adam / k_train_reduce add the slices in FP64 (no atomics, no
+// zeroing; the same result every time, and with two chunks the per-layer
+// kernels' bit for bit).  A layer's blocks go over the XCDs by slice (xcd_run):
+// with eight slices every XCD's L2 reads one (2.8 of the surrogate's 22 MB)
+// instead of all, the one whose rows k_train_rows wrote there.  A chunk is staged 64
+// rows at a time through two LDS buffers (32 and zeros at its end).  The tiles of
 // a layer's first input column block also sum their gradient rows: the biases.
-constexpr int DW_P = 64 + 8, DW_SLICES = 8;
+constexpr int DW_P = 64 + 8, DW_SLICES = 16;
 struct DwArgs {
-    int L, batch, ld, kchunk, slices;
+    int L, batch, ld;
     size_t n_pad;
-    int tile0[TR_MAX_LAYERS + 2];          // first tile of layer l
+    int block0[TR_MAX_LAYERS + 2];         // first block of layer l
+    int chunks[TR_MAX_LAYERS + 1], kc[TR_MAX_LAYERS + 1], slices[TR_MAX_LAYERS + 1];
     int mtiles[TR_MAX_LAYERS + 1], cols[TR_MAX_LAYERS + 1];
     const bf16 *dz[TR_MAX_LAYERS + 1], *in[TR_MAX_LAYERS + 1];
     size_t woff[TR_MAX_LAYERS + 1], boff[TR_MAX_LAYERS + 1];
@@ -286,14 +291,14 @@ __global__ void __launch_bounds__(256) k_train_dw(const DwArgs g)
 {
     __shared__ __attribute__((aligned(16))) bf16 As[2][64 * DW_P];
     __shared__ __attribute__((aligned(16))) bf16 Bs[2][64 * DW_P];
-    const int slice = blockIdx.x % g.slices, at = blockIdx.x / g.slices;
     int l = 0;
-    while (at >= g.tile0[l + 1]) ++l;
-    const int tile = at - g.tile0[l];
+    while ((int)blockIdx.x >= g.block0[l + 1]) ++l;
+    const int slices = g.slices[l], chunks = g.chunks[l], kc = g.kc[l], blocks = g.block0[l + 1] - g.block0[l];
+    const int at = xcd_run(blockIdx.x - g.block0[l], blocks), tiles = blocks / slices, slice = at / tiles, tile = at % tiles;
     const int m0 = (tile % g.mtiles[l]) * 64, n0 = (tile / g.mtiles[l]) * 64;
     const int cols = g.cols[l];
     const int t = threadIdx.x, lane = t & 63, wave = t >> 6, wm = wave >> 1, wn = wave & 1;
-    const int kb = slice * g.kchunk, ke = min(g.batch, kb + g.kchunk);
+    const int kb = slice * chunks / slices * kc, ke = min(g.batch, (slice + 1) * chunks / slices * kc);
     // each thread moves 2 x 16 B of either operand per stage: rows t / 8 and + 32
     const int lr = t >> 3, lk = (t & 7) * 8;
     const bf16 *A = g.dz[l] + (size_t)(m0 + lr) * g.ld + lk;
@@ -304,29 +309,39 @@ __global__ void __launch_bounds__(256) k_train_dw(const DwArgs g)
     bf16x8 ra0 = *reinterpret_cast<const bf16x8 *>(A + kb), ra1 = *reinterpret_cast<const bf16x8 *>(A1 + kb);
     bf16x8 rb0 = *reinterpret_cast<const bf16x8 *>(B + kb), rb1 = *reinterpret_cast<const bf16x8 *>(B1 + kb);
     bf16 *const sa = &As[0][lr * DW_P + lk], *const sb = &Bs[0][lr * DW_P + lk];
-    float bs0 = 0.f, bs1 = 0.f;
+    double bs0 = 0.0, bs1 = 0.0;
     const bool bias = n0 == 0;
-    f32x16 acc = {};
-    int buf = 0;
-    for (int k = kb; k < ke; k += 64, buf ^= 1) {
+    f32x16 acc = {}, sum = {};
+    for (int k = kb, ce = min(ke, kb + kc), buf = 0;; buf ^= 1) {   // ce: the chunk's end
         // stage k's rows; this buffer was read last before the barrier of the turn between
+        const int rows = ce - k;           // 32 left of the chunk (a multiple of 32): the others as zeros
+        if (rows < 64 && lk >= rows) ra0 = ra1 = rb0 = rb1 = bf16x8{};
         const int o = buf * 64 * DW_P;
         *reinterpret_cast<bf16x8 *>(sa + o) = ra0;
         *reinterpret_cast<bf16x8 *>(sa + o + 32 * DW_P) = ra1;
         *reinterpret_cast<bf16x8 *>(sb + o) = rb0;
         *reinterpret_cast<bf16x8 *>(sb + o + 32 * DW_P) = rb1;
         if (bias) {
+            float s0 = 0.f, s1 = 0.f;
 #pragma unroll
             for (int j = 0; j < 8; ++j) {
-                bs0 += (float)ra0[j];
-                bs1 += (float)ra1[j];
+                s0 += (float)ra0[j];
+                s1 += (float)ra1[j];
             }
+            bs0 += (double)s0;
+            bs1 += (double)s1;
         }
-        const int kn = min(k + 64, ke - 64);
-        ra0 = *reinterpret_cast<const bf16x8 *>(A + kn);
-        ra1 = *reinterpret_cast<const bf16x8 *>(A1 + kn);
-        rb0 = *reinterpret_cast<const bf16x8 *>(B + kn);
-        rb1 = *reinterpret_cast<const bf16x8 *>(B1 + kn);
+        const int kn = min(k + 64, ce);
+        const bool more = kn < ke;
+        {
+            // (rows past the chunk's or the batch's end may be among them: the next
+            // chunk's or the arrays' pad)
+            const int kl = more ? kn : k;
+            ra0 = *reinterpret_cast<const bf16x8 *>(A + kl);
+            ra1 = *reinterpret_cast<const bf16x8 *>(A1 + kl);
+            rb0 = *reinterpret_cast<const bf16x8 *>(B + kl);
+            rb1 = *reinterpret_cast<const bf16x8 *>(B1 + kl);
+        }
         __syncthreads();
         const bf16 *a = &As[buf][(wm * 32 + (lane & 31)) * DW_P + (lane >> 5) * 8];
         const bf16 *b = &Bs[buf][(wn * 32 + (lane & 31)) * DW_P + (lane >> 5) * 8];
@@ -334,6 +349,13 @@ __global__ void __launch_bounds__(256) k_train_dw(const DwArgs g)
         for (int s = 0; s < 4; ++s)
             acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(*reinterpret_cast<const bf16x8 *>(a + 16 * s),
                                                           *reinterpret_cast<const bf16x8 *>(b + 16 * s), acc, 0, 0, 0);
+        if (kn == ce) {                    // the chunk is complete
+            sum += acc;
+            acc = f32x16{};
+            ce = min(ke, ce + kc);
+        }
+        if (!more) break;
+        k = kn;
     }
     float *out = g.part + (size_t)slice * g.n_pad;
     const int n = n0 + wn * 32 + (lane & 31);
@@ -341,7 +363,7 @@ __global__ void __launch_bounds__(256) k_train_dw(const DwArgs g)
         float *o = out + g.woff[l] + n;
 #pragma unroll
         for (int r = 0; r < 16; ++r)
-            o[(size_t)(m0 + wm * 32 + (r >> 2) * 8 + (lane >> 5) * 4 + (r & 3)) * cols] = acc[r];
+            o[(size_t)(m0 + wm * 32 + (r >> 2) * 8 + (lane >> 5) * 4 + (r & 3)) * cols] = sum[r];
     }
     if (bias) {
 #pragma unroll
@@ -350,8 +372,8 @@ __global__ void __launch_bounds__(256) k_train_dw(const DwArgs g)
             bs1 += __shfl_xor(bs1, d, 64);
         }
         if ((t & 7) == 0) {
-            out[g.boff[l] + m0 + lr] = bs0;
-            out[g.boff[l] + m0 + lr + 32] = bs1;
+            out[g.boff[l] + m0 + lr] = (float)bs0;
+            out[g.boff[l] + m0 + lr + 32] = (float)bs1;
         }
     }
 }
@@ -409,6 +431,19 @@ __device__ __forceinline__ void loss_of(const float *lpart, int nb, int rows, fl
     if (threadIdx.x == 0) *loss = red[0] / rows;
 }
 
+// The slices' partial sums (k_train_dw)
+struct GradParts {
+    const float *part;                     // [slice][n_pad]
+    int slices[TR_MAX_LAYERS + 1];
+};
+__device__ __forceinline__ float grad_sum(const GradParts &gp, size_t n_pad, int l, size_t i)
+{
+    double g = 0.0;
+#pragma unroll 4
+    for (int s = 0; s < gp.slices[l]; ++s) g += (double)gp.part[(size_t)s * n_pad + i];
+    return (float)g;
+}
+
 // Gradient = sum of the slices' partial sums, then Adam (decoupled weight
 // decay) on the FP32 parameters and the bf16 operand copies.  A block takes a
 // 32 x 32 patch of a layer's weights, four columns per thread, and turns it in
@@ -419,8 +454,7 @@ struct AdamArgs {
     ParamMap m;
     int patch0[TR_MAX_LAYERS + 2];         // first patch of layer l; [L + 1]: number of patches
     int bias0[TR_MAX_LAYERS + 2];          // first bias block of layer l
-    const float *part;
-    int slices;
+    GradParts g;
     float *p, *mo, *vo;
     float lr_t, b1, b2, eps, wd_lr;
     bf16 *wf, *wt;
@@ -450,8 +484,7 @@ __global__ void __launch_bounds__(256) k_train_adam(const AdamArgs a)
         const int r = (k - a.bias0[l]) * 256 + t;
         if (r >= m.rows[l]) return;
         const size_t i = m.boff[l] + r;
-        float g = 0.f;
-        for (int s = 0; s < a.slices; ++s) g += a.part[(size_t)s * m.n_pad + i];
+        const float g = grad_sum(a.g, m.n_pad, l, i);
         float p = a.p[i], mi = a.mo[i], vi = a.vo[i];
         adam_step(a, g, p, mi, vi);
         a.p[i] = p; a.mo[i] = mi; a.vo[i] = vi;
@@ -463,11 +496,13 @@ __global__ void __launch_bounds__(256) k_train_adam(const AdamArgs a)
     const int r = t >> 3, c = (t & 7) * 4;                // this thread's row and columns of the patch
     const int row = pr * 32 + r, col = pc * 32 + c;
     const size_t i = m.woff[l] + ((size_t)row << m.lgcol[l]) + col;
-    float4 g = make_float4(0.f, 0.f, 0.f, 0.f);
-    for (int s = 0; s < a.slices; ++s) {
-        const float4 d = *reinterpret_cast<const float4 *>(a.part + (size_t)s * m.n_pad + i);
-        g.x += d.x; g.y += d.y; g.z += d.z; g.w += d.w;
+    double gx = 0.0, gy = 0.0, gz = 0.0, gw = 0.0;
+#pragma unroll 4
+    for (int s = 0; s < a.g.slices[l]; ++s) {
+        const float4 d = *reinterpret_cast<const float4 *>(a.g.part + (size_t)s * m.n_pad + i);
+        gx += (double)d.x; gy += (double)d.y; gz += (double)d.z; gw += (double)d.w;
     }
+    const float4 g = make_float4((float)gx, (float)gy, (float)gz, (float)gw);
     float4 p = *reinterpret_cast<float4 *>(a.p + i), mi = *reinterpret_cast<float4 *>(a.mo + i),
            vi = *reinterpret_cast<float4 *>(a.vo + i);
     // padding rows and columns stay zero
@@ -497,16 +532,13 @@ __global__ void __launch_bounds__(256) k_train_adam(const AdamArgs a)
 }
 
 // gradient array and loss without an update
-__global__ void __launch_bounds__(256) k_train_reduce(const ParamMap m, const float *part, int slices, float *gr,
-                                                      const float *lpart, int nb, int rows, float *loss)
+__global__ void __launch_bounds__(256) k_train_reduce(const ParamMap m, const GradParts gp, float *gr, const float *lpart, int nb, int rows, float *loss)
 {
     if (blockIdx.x == 0) loss_of(lpart, nb, rows, loss);
     const size_t i = blockIdx.x * (size_t)256 + threadIdx.x;
     if (i >= m.n_pad) return;
-    float g = 0.f;
-    if (param_at(m, i).real)
-        for (int s = 0; s < slices; ++s) g += part[(size_t)s * m.n_pad + i];
-    gr[i] = g;
+    const ParamAt a = param_at(m, i);
+    gr[i] = a.real ? grad_sum(gp, m.n_pad, a.l, i) : 0.f;
 }
 
 // every bf16 copy of the weights from the FP32 parameters (wb: row-major; wf, wt: operands, may be null)
