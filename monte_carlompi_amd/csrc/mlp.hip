@@ -399,22 +399,33 @@ __global__ void k_fill_f32(float *p, size_t n, float v)
         p[i] = v;
 }
 
-// Adam (decoupled weight decay) over the padded parameter buffer, refreshing
-// the bf16 copies of weights; mask zeroes updates of padding.
+// Adam (decoupled weight decay) on one parameter.  Which of the two products of
+// a moment goes into the fused multiply-add is written out: left to the
+// compiler it differed between the kernels that call this, and with it the
+// moments' last bits.
+struct AdamCoef {
+    float lr_t, b1, b2, eps, wd_lr;
+};
+__device__ __forceinline__ void adam_step(const AdamCoef &a, float g, float &p, float &m, float &v)
+{
+#pragma clang fp contract(off)
+    m = fmaf(1.f - a.b1, g, a.b1 * m);
+    v = fmaf((1.f - a.b2) * g, g, a.b2 * v);
+    p = fmaf(-a.wd_lr, p, p - a.lr_t * m / (sqrtf(v) + a.eps));
+}
+
+// Adam over the padded parameter buffer, refreshing the bf16 copies of weights;
+// mask zeroes updates of padding.
 __global__ void k_adam(float *p, const float *gr, float *m, float *v, const uint8_t *mask, size_t n,
-                       float lr_t, float b1, float b2, float eps, float wd_lr, bf16 *pb, const int64_t *pb_index)
+                       AdamCoef a, bf16 *pb, const int64_t *pb_index)
 {
     for (size_t i = blockIdx.x * (size_t)blockDim.x + threadIdx.x; i < n; i += (size_t)gridDim.x * blockDim.x) {
         if (!mask[i]) continue;
-        const float g = gr[i];
-        const float mi = b1 * m[i] + (1.f - b1) * g;
-        const float vi = b2 * v[i] + (1.f - b2) * g * g;
-        m[i] = mi;
-        v[i] = vi;
-        const float np_ = p[i] - lr_t * mi / (sqrtf(vi) + eps) - wd_lr * p[i];
-        p[i] = np_;
+        float pi = p[i], mi = m[i], vi = v[i];
+        adam_step(a, gr[i], pi, mi, vi);
+        p[i] = pi; m[i] = mi; v[i] = vi;
         const int64_t j = pb_index[i];
-        if (j >= 0) pb[j] = (bf16)np_;
+        if (j >= 0) pb[j] = (bf16)pi;
     }
 }
 
@@ -1151,13 +1162,13 @@ int mcs_mlp_train_steps(mcs_mlp *c, const int32_t *idx, int32_t n_steps, int32_t
         c->didx_cap = ni;
     }
     MCHK(c, hipMemcpy(c->didx, idx, sizeof(int32_t) * ni, hipMemcpyHostToDevice));
+    AdamCoef coef{0.f, a->beta1, a->beta2, a->eps, a->lr * a->weight_decay};   // lr_t: the step's
     AdamArgs adam;
     memset(&adam, 0, sizeof adam);
     int adam_blocks = 0;
     if (c->train_rows) {
         adam.m = c->pm;
         adam.p = c->p; adam.mo = c->m; adam.vo = c->v;
-        adam.b1 = a->beta1; adam.b2 = a->beta2; adam.eps = a->eps; adam.wd_lr = a->lr * a->weight_decay;
         adam.wf = c->wf; adam.wt = c->wt;
         adam.lpart = c->lpart; adam.nb = batch / TR_ROWS; adam.rows = batch;
         int patches = 0, bias = 0;
@@ -1175,10 +1186,10 @@ int mcs_mlp_train_steps(mcs_mlp *c, const int32_t *idx, int32_t n_steps, int32_t
         const int32_t *rows = c->didx + (size_t)s * batch;
         float *const loss_out = c->loss + 1 + s;   // step s's loss in loss[1 + s]
         const int t = a->step + s + 1;
-        const float lr_t = a->lr * std::sqrt(1.f - std::pow(a->beta2, (float)t)) / (1.f - std::pow(a->beta1, (float)t));
+        coef.lr_t = a->lr * std::sqrt(1.f - std::pow(a->beta2, (float)t)) / (1.f - std::pow(a->beta1, (float)t));
         if (c->train_rows) {
             adam.g = rows_backward(c, c->xd, c->td, c->n_data, rows, batch);
-            adam.lr_t = lr_t;
+            adam.c = coef;
             adam.loss = loss_out;
             hipLaunchKernelGGL(k_train_adam, dim3(adam_blocks), dim3(256), 0, c->stream, adam);
             continue;
@@ -1188,7 +1199,7 @@ int mcs_mlp_train_steps(mcs_mlp *c, const int32_t *idx, int32_t n_steps, int32_t
         forward_pass(c, batch);
         backward_pass(c, batch, loss_out);
         hipLaunchKernelGGL(k_adam, dim3(1024), dim3(256), 0, c->stream, c->p, c->gr, c->m, c->v, c->mask, c->n_pad,
-                           lr_t, a->beta1, a->beta2, a->eps, a->lr * a->weight_decay, c->wb, c->pb_index);
+                           coef, c->wb, c->pb_index);
     }
     if (c->fused) pack_serve(c);          // the copy that inference reads
     MCHK(c, hipGetLastError());

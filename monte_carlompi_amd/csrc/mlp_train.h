@@ -456,20 +456,12 @@ struct AdamArgs {
     int bias0[TR_MAX_LAYERS + 2];          // first bias block of layer l
     GradParts g;
     float *p, *mo, *vo;
-    float lr_t, b1, b2, eps, wd_lr;
+    AdamCoef c;
     bf16 *wf, *wt;
     const float *lpart;
     int nb, rows;
     float *loss;
 };
-
-__device__ __forceinline__ float adam_step(const AdamArgs &a, float g, float &p, float &m, float &v)
-{
-    m = a.b1 * m + (1.f - a.b1) * g;
-    v = a.b2 * v + (1.f - a.b2) * g * g;
-    p = p - a.lr_t * m / (sqrtf(v) + a.eps) - a.wd_lr * p;
-    return p;
-}
 
 __global__ void __launch_bounds__(256) k_train_adam(const AdamArgs a)
 {
@@ -486,7 +478,7 @@ __global__ void __launch_bounds__(256) k_train_adam(const AdamArgs a)
         const size_t i = m.boff[l] + r;
         const float g = grad_sum(a.g, m.n_pad, l, i);
         float p = a.p[i], mi = a.mo[i], vi = a.vo[i];
-        adam_step(a, g, p, mi, vi);
+        adam_step(a.c, g, p, mi, vi);
         a.p[i] = p; a.mo[i] = mi; a.vo[i] = vi;
         return;
     }
@@ -507,10 +499,10 @@ __global__ void __launch_bounds__(256) k_train_adam(const AdamArgs a)
            vi = *reinterpret_cast<float4 *>(a.vo + i);
     // padding rows and columns stay zero
     const bool in = row < m.rows[l];
-    if (in && col < m.cols[l]) adam_step(a, g.x, p.x, mi.x, vi.x);
-    if (in && col + 1 < m.cols[l]) adam_step(a, g.y, p.y, mi.y, vi.y);
-    if (in && col + 2 < m.cols[l]) adam_step(a, g.z, p.z, mi.z, vi.z);
-    if (in && col + 3 < m.cols[l]) adam_step(a, g.w, p.w, mi.w, vi.w);
+    if (in && col < m.cols[l]) adam_step(a.c, g.x, p.x, mi.x, vi.x);
+    if (in && col + 1 < m.cols[l]) adam_step(a.c, g.y, p.y, mi.y, vi.y);
+    if (in && col + 2 < m.cols[l]) adam_step(a.c, g.z, p.z, mi.z, vi.z);
+    if (in && col + 3 < m.cols[l]) adam_step(a.c, g.w, p.w, mi.w, vi.w);
     *reinterpret_cast<float4 *>(a.p + i) = p;
     *reinterpret_cast<float4 *>(a.mo + i) = mi;
     *reinterpret_cast<float4 *>(a.vo + i) = vi;

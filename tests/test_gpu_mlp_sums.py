@@ -56,3 +56,26 @@ def test_chunks_in_another_order_only(monkeypatch, n_in, L, n_out, batch):
     for l, ((Wa, ca), (Wb, cb)) in enumerate(zip(a.unflatten(ga), b.unflatten(gb))):
         assert off(Wa, Wb) < 1e-6 and off(ca, cb) < 1e-6, (l, off(Wa, Wb), off(ca, cb))
     a.close(); b.close()
+
+
+@pytest.mark.parametrize('n_in,L,n_out', [(9, 4, 651), (5, 1, 65)])
+def test_adam_with_moments_rounds_as_the_per_layer_path(monkeypatch, n_in, L, n_out):
+    """The first steps with a learning rate of zero fill the moments from
+    gradients that both paths have bit for bit (the parameters stay); the step
+    after them then gives the same weights only if the moments' expressions
+    round alike."""
+    layers, x, t, w = inputs(n_in, L, n_out, 256)
+    nets_ = nets(monkeypatch, (n_in, 256, L, n_out, 64), layers)
+    got = []
+    for net in nets_:
+        net.set_dataset(x, t)
+        idx = np.arange(256, dtype=np.int32)
+        net.train_steps(idx[:192], 64, w, lr=0.0)
+        np.testing.assert_array_equal(net.get_params(), net.flatten(layers))
+        net.train_steps(idx[192:], 64, w, lr=1e-2, weight_decay=1e-2)
+        got.append(net.unflatten(net.get_params()))
+    for l, ((Wa, ca), (Wb, cb), (W0, c0)) in enumerate(zip(*got, layers)):
+        np.testing.assert_array_equal(Wa, Wb, err_msg='layer %d' % l)
+        assert np.mean(Wa != W0) > 0.9
+    for net in nets_:
+        net.close()
