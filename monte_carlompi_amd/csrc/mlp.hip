@@ -876,7 +876,9 @@ int mcs_mlp_create(int device, const mcs_mlp_dims *dims, mcs_mlp **out)
         hipMemcpy(c->pb_index, pbi.data(), off * sizeof(int64_t), hipMemcpyHostToDevice) != hipSuccess ||
         hipMemset(c->p, 0, off * 4) != hipSuccess || hipMemset(c->m, 0, off * 4) != hipSuccess ||
         hipMemset(c->v, 0, off * 4) != hipSuccess || hipMemset(c->gr, 0, off * 4) != hipSuccess ||
-        hipMemset(c->wb, 0, woff * 2) != hipSuccess) {
+        hipMemset(c->wb, 0, woff * 2) != hipSuccess || (c->ws && hipMemset(c->ws, 0, woff * 2) != hipSuccess) ||
+        (c->wf && hipMemset(c->wf, 0, woff * 2) != hipSuccess) || (c->wt && hipMemset(c->wt, 0, woff * 2) != hipSuccess) ||
+        hipStreamSynchronize(nullptr) != hipSuccess) {   // (c->stream does not wait for the null stream)
         mcs_mlp_destroy(c);
         return MCS_ERR_HIP;
     }
