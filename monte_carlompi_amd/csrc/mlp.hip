@@ -551,7 +551,8 @@ static void gemm_fwd(mcs_mlp *c, const GemmArgs &g)
     hipLaunchKernelGGL((k_gemm_fwd<EPI>), grid, dim3(256), 0, c->stream, g);
 }
 
-// Inference of a 256-wide network, any number of rows in one launch: x device
+// Inference of a 256-wide network in one launch, or in passes of 2^28 rows (a
+// launch holds at most 2^32 threads: 2^30 rows at four threads each): x device
 // rows (raw case inputs if `snow`, else n_in features), outputs [rows][n_out]
 // into `y` (through the output transform if `exp_out`).  Rows per block: 128
 // where that fills the CUs twice (operands from L2 and LDS are then shared by
@@ -564,6 +565,12 @@ static void gemm_fwd(mcs_mlp *c, const GemmArgs &g)
 // in passes of max_batch rows: 65, 69, 75, 139 and 2112).
 static void serve_rows(mcs_mlp *c, const float *x, int64_t rows, float *y, bool snow, bool exp_out)
 {
+    constexpr int64_t PASS = int64_t(1) << 28;
+    for (; rows > PASS; rows -= PASS) {
+        serve_rows(c, x, PASS, y, snow, exp_out);
+        x += PASS * (snow ? 5 : c->d.n_in);
+        y += PASS * c->d.n_out;
+    }
     ServeArgs g;
     memset(&g, 0, sizeof g);
     g.x = x; g.rows = rows; g.snow = snow; g.n_in = c->d.n_in;
