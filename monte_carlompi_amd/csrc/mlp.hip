@@ -457,13 +457,12 @@ struct mcs_mlp {
     float *p = nullptr, *gr = nullptr, *m = nullptr, *v = nullptr;
     uint8_t *mask = nullptr;
     int64_t *pb_index = nullptr;
-    bf16 *wb = nullptr;
+    bf16 *wb = nullptr;              // row-major bf16 weights (the per-layer kernels')
     // activations (max_batch rows)
     bf16 *X = nullptr, *dY = nullptr, *dZa = nullptr, *dZb = nullptr;
     std::vector<float *> Z;
     std::vector<bf16 *> A;
     float *Y = nullptr, *T = nullptr, *w = nullptr, *yout = nullptr, *xin = nullptr, *loss = nullptr;
-    int32_t *idx = nullptr;
     float *lpart = nullptr;          // k_loss: per-block partial sums (LOSS_BLOCKS)
     // inference through k_mlp_serve (256-wide networks) and its operand copy of
     // the weights
@@ -713,7 +712,7 @@ static void backward_pass(mcs_mlp *c, int rows, float *loss_out)
 static void pack_weights(mcs_mlp *c)
 {
     hipLaunchKernelGGL(k_pack_weights, dim3((unsigned)((c->n_pad + 255) / 256)), dim3(256), 0, c->stream, c->pm, c->p,
-                       c->wb, c->wf, c->wt);
+                       c->wf, c->wt);
 }
 
 // Slices of the batch (whole chunks) for a layer's weight gradients: of eight
@@ -833,9 +832,12 @@ int mcs_mlp_create(int device, const mcs_mlp_dims *dims, mcs_mlp **out)
     }
     c->n_pad = off; c->n_wb = woff; c->n_flat = flat;
     const size_t MB = dims->max_batch;
-    std::vector<uint8_t> mask(off, 0);
-    std::vector<int64_t> pbi(off, -1);
+    // what only the per-layer kernels read
+    const bool layered = !c->train_rows;
+    std::vector<uint8_t> mask(layered ? off : 0, 0);
+    std::vector<int64_t> pbi(layered ? off : 0, -1);
     for (const Layer &ly : c->layers) {
+        if (!layered) break;
         for (int r = 0; r < ly.rows; ++r) {
             for (int k = 0; k < ly.cols; ++k) {
                 mask[ly.w_off + (size_t)r * ly.pcol + k] = 1;
@@ -847,13 +849,10 @@ int mcs_mlp_create(int device, const mcs_mlp_dims *dims, mcs_mlp **out)
     }
     bool ok = dalloc(&c->p, off) == hipSuccess && dalloc(&c->gr, off) == hipSuccess &&
               dalloc(&c->m, off) == hipSuccess && dalloc(&c->v, off) == hipSuccess &&
-              dalloc(&c->mask, off) == hipSuccess && dalloc(&c->pb_index, off) == hipSuccess &&
-              dalloc(&c->wb, woff) == hipSuccess && dalloc(&c->X, (MB + LD_PAD) * K0) == hipSuccess &&
-              dalloc(&c->dY, (MB + LD_PAD) * c->np) == hipSuccess && dalloc(&c->dZa, MB * H) == hipSuccess &&
-              dalloc(&c->dZb, MB * H) == hipSuccess && dalloc(&c->Y, MB * c->np) == hipSuccess &&
+              dalloc(&c->X, (MB + LD_PAD) * K0) == hipSuccess && dalloc(&c->dY, (MB + LD_PAD) * c->np) == hipSuccess &&
               dalloc(&c->T, MB * c->np) == hipSuccess && dalloc(&c->w, c->np) == hipSuccess &&
               dalloc(&c->yout, MB * dims->n_out) == hipSuccess && dalloc(&c->xin, MB * dims->n_in) == hipSuccess &&
-              dalloc(&c->loss, 1024) == hipSuccess && dalloc(&c->idx, MB) == hipSuccess &&
+              dalloc(&c->loss, 1024) == hipSuccess &&
               dalloc(&c->lpart, std::max<size_t>(LOSS_BLOCKS, MB / TR_ROWS)) == hipSuccess;
     for (int l = 0; ok && l < L; ++l) {
         float *z = nullptr;
@@ -862,6 +861,10 @@ int mcs_mlp_create(int device, const mcs_mlp_dims *dims, mcs_mlp **out)
         c->Z.push_back(z);
         c->A.push_back(a);
     }
+    if (ok && layered)
+        ok = dalloc(&c->mask, off) == hipSuccess && dalloc(&c->pb_index, off) == hipSuccess &&
+             dalloc(&c->wb, woff) == hipSuccess && dalloc(&c->dZa, MB * H) == hipSuccess &&
+             dalloc(&c->dZb, MB * H) == hipSuccess && dalloc(&c->Y, MB * c->np) == hipSuccess;
     if (ok && c->fused) ok = dalloc(&c->ws, woff) == hipSuccess;
     if (ok && c->train_rows) {
         ok = dalloc(&c->wf, woff) == hipSuccess && dalloc(&c->wt, woff) == hipSuccess &&
@@ -879,12 +882,11 @@ int mcs_mlp_create(int device, const mcs_mlp_dims *dims, mcs_mlp **out)
         mcs_mlp_destroy(c);
         return MCS_ERR_NOMEM;
     }
-    if (hipMemcpy(c->mask, mask.data(), off, hipMemcpyHostToDevice) != hipSuccess ||
-        hipMemcpy(c->pb_index, pbi.data(), off * sizeof(int64_t), hipMemcpyHostToDevice) != hipSuccess ||
-        hipMemset(c->p, 0, off * 4) != hipSuccess || hipMemset(c->m, 0, off * 4) != hipSuccess ||
-        hipMemset(c->v, 0, off * 4) != hipSuccess || hipMemset(c->gr, 0, off * 4) != hipSuccess ||
-        hipMemset(c->wb, 0, woff * 2) != hipSuccess || (c->ws && hipMemset(c->ws, 0, woff * 2) != hipSuccess) ||
-        (c->wf && hipMemset(c->wf, 0, woff * 2) != hipSuccess) || (c->wt && hipMemset(c->wt, 0, woff * 2) != hipSuccess) ||
+    const auto clear = [](void *p, size_t bytes) { return !p || hipMemset(p, 0, bytes) == hipSuccess; };
+    if ((layered && (hipMemcpy(c->mask, mask.data(), off, hipMemcpyHostToDevice) != hipSuccess ||
+                     hipMemcpy(c->pb_index, pbi.data(), off * sizeof(int64_t), hipMemcpyHostToDevice) != hipSuccess)) ||
+        !clear(c->p, off * 4) || !clear(c->m, off * 4) || !clear(c->v, off * 4) || !clear(c->gr, off * 4) ||
+        !clear(c->wb, woff * 2) || !clear(c->ws, woff * 2) || !clear(c->wf, woff * 2) || !clear(c->wt, woff * 2) ||
         hipStreamSynchronize(nullptr) != hipSuccess) {   // (c->stream does not wait for the null stream)
         mcs_mlp_destroy(c);
         return MCS_ERR_HIP;
@@ -900,7 +902,7 @@ int mcs_mlp_destroy(mcs_mlp *c)
     if (c->stream) (void)hipStreamSynchronize(c->stream);
     c->copier.release();
     void *bufs[] = {c->p, c->gr, c->m, c->v, c->mask, c->pb_index, c->wb, c->X, c->dY, c->dZa, c->dZb,
-                    c->Y, c->T, c->w, c->yout, c->xin, c->loss, c->idx, c->xd, c->td,
+                    c->Y, c->T, c->w, c->yout, c->xin, c->loss, c->xd, c->td,
                     c->fmu, c->fsd, c->oscale, c->oshift, c->ooff, c->lpart, c->ws, c->wf, c->wt, c->part, c->didx};
     for (void *b : bufs) if (b) (void)hipFree(b);
     for (float *z : c->Z) if (z) (void)hipFree(z);
@@ -929,19 +931,19 @@ int mcs_mlp_set_params(mcs_mlp *c, const float *params, int64_t n)
         if (!std::isfinite(params[i])) return merr(c, MCS_ERR_ARG, "parameter %lld is not finite", (long long)i);
     (void)hipSetDevice(c->device);
     std::vector<float> pad(c->n_pad, 0.f);
-    std::vector<bf16> wb(c->n_wb, (bf16)0.f);
+    std::vector<bf16> wb(c->wb ? c->n_wb : 0, (bf16)0.f);
     size_t k = 0;
     for (const Layer &ly : c->layers) {
         for (int r = 0; r < ly.rows; ++r)
             for (int q = 0; q < ly.cols; ++q) {
                 pad[ly.w_off + (size_t)r * ly.pcol + q] = params[k];
-                wb[ly.wb_off + (size_t)r * ly.pcol + q] = (bf16)params[k];
+                if (c->wb) wb[ly.wb_off + (size_t)r * ly.pcol + q] = (bf16)params[k];
                 ++k;
             }
         for (int r = 0; r < ly.rows; ++r) pad[ly.b_off + r] = params[k++];
     }
     MCHK(c, hipMemcpy(c->p, pad.data(), pad.size() * 4, hipMemcpyHostToDevice));
-    MCHK(c, hipMemcpy(c->wb, wb.data(), wb.size() * 2, hipMemcpyHostToDevice));
+    if (c->wb) MCHK(c, hipMemcpy(c->wb, wb.data(), wb.size() * 2, hipMemcpyHostToDevice));
     MCHK(c, hipMemset(c->m, 0, c->n_pad * 4));
     MCHK(c, hipMemset(c->v, 0, c->n_pad * 4));
     if (c->train_rows) pack_weights(c);

@@ -533,16 +533,14 @@ __global__ void __launch_bounds__(256) k_train_reduce(const ParamMap m, const Gr
     gr[i] = a.real ? grad_sum(gp, m.n_pad, a.l, i) : 0.f;
 }
 
-// every bf16 copy of the weights from the FP32 parameters (wb: row-major; wf, wt: operands, may be null)
-__global__ void __launch_bounds__(256) k_pack_weights(const ParamMap m, const float *p, bf16 *wb, bf16 *wf, bf16 *wt)
+// the bf16 operand copies of the weights from the FP32 parameters
+__global__ void __launch_bounds__(256) k_pack_weights(const ParamMap m, const float *p, bf16 *wf, bf16 *wt)
 {
     const size_t i = blockIdx.x * (size_t)256 + threadIdx.x;
     if (i >= m.n_pad) return;
     const ParamAt a = param_at(m, i);
     if (!a.weight) return;
-    const float v = p[i];
-    wb[m.wboff[a.l] + (i - m.woff[a.l])] = (bf16)v;
-    put_tiles(m, a, v, wf, wt);
+    put_tiles(m, a, p[i], wf, wt);
 }
 
 }  // namespace mlp

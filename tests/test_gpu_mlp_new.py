@@ -62,3 +62,22 @@ def test_new_network_is_zero(monkeypatch, dims):
         np.testing.assert_array_equal(W, 0.0)
     np.testing.assert_allclose(np.abs(p[-1][1]), 1e-3, rtol=1e-3)           # the first step is the rate's size
     net.close()
+
+
+def test_no_buffers_for_kernels_that_never_run(monkeypatch):
+    """The row kernels' network at the largest batch: inputs 7 MB, targets
+    and outputs 184 + 171, gradients of both 92, pre-activations and activations
+    4 x (67 + 34), parameters and their sums 40: 0.90 GB.  The per-layer kernels'
+    outputs and gradients (0.26 GB) are not among it."""
+    import torch
+    from monte_carlompi_amd.mlp import Mlp
+    used = {}
+    for layered in ('0', '1'):
+        monkeypatch.setenv('MCS_MLP_LAYERED', layered)
+        torch.cuda.synchronize()
+        free = torch.cuda.mem_get_info()[0]
+        net = Mlp(9, 256, 4, 651, 65536)
+        used[layered] = free - torch.cuda.mem_get_info()[0]
+        net.close()
+    print('bytes', used)
+    assert 0.8e9 < used['0'] < 0.98e9
