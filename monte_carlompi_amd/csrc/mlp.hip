@@ -446,7 +446,7 @@ struct Layer {
 };
 
 struct mcs_mlp {
-    int device = 0;
+    int device = 0, cus = 0;
     mcs_mlp_dims d{};
     int np = 0;  // padded outputs
     hipStream_t stream = nullptr;
@@ -581,9 +581,9 @@ static void serve_rows(mcs_mlp *c, const float *x, int64_t rows, float *y, bool 
     const auto go = [&](auto kernel, int R) {
         hipLaunchKernelGGL(kernel, dim3((unsigned)((rows + R - 1) / R)), dim3(SV_WAVES * 64), 0, c->stream, g);
     };
-    if (rows <= 32 * 256)
+    if (rows <= 32 * (int64_t)c->cus)
         exp_out ? go(k_mlp_serve<1, 16, 2, true>, 32) : go(k_mlp_serve<1, 16, 2, false>, 32);
-    else if (rows <= 64 * 512)
+    else if (rows <= 64 * 2 * (int64_t)c->cus)
         exp_out ? go(k_mlp_serve<2, 4, 4, true>, 64) : go(k_mlp_serve<2, 4, 4, false>, 64);
     else
         exp_out ? go(k_mlp_serve<4, 4, 4, true>, 128) : go(k_mlp_serve<4, 4, 4, false>, 128);
@@ -812,7 +812,8 @@ int mcs_mlp_create(int device, const mcs_mlp_dims *dims, mcs_mlp **out)
     }
     c->train_rows = c->fused && dims->hidden == TR_H && dims->n_hidden_layers <= TR_MAX_LAYERS && c->np <= TR_MAX_NP;
     if (hipSetDevice(device) != hipSuccess || hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking) != hipSuccess ||
-        hipEventCreate(&c->e0) != hipSuccess || hipEventCreate(&c->e1) != hipSuccess) {
+        hipEventCreate(&c->e0) != hipSuccess || hipEventCreate(&c->e1) != hipSuccess ||
+        hipDeviceGetAttribute(&c->cus, hipDeviceAttributeMultiprocessorCount, device) != hipSuccess) {
         mcs_mlp_destroy(c);
         return MCS_ERR_HIP;
     }
