@@ -1077,6 +1077,7 @@ struct mcs_ctx {
     hipEvent_t ev0 = nullptr, ev1 = nullptr;
     char err[512] = {0};
     mcs_launch launch{256, 4, 2048, 8, 16};
+    int tune_chunk = 0;             // > 0: mcs_autotune times a part of a queue walk, whose chunk this is
     // host copies
     std::vector<mcs_case> cases;
     std::vector<mcs_band> bands;
@@ -1655,6 +1656,8 @@ static int64_t count_chunks(const mcs_ctx *c, int chunk)
 //   records do not depend on the shape (coop_live 0, polarised, replay) then
 //   shrink their chunks to one per block (500,000 photons at the default
 //   shape, coop_live 0: kernel 2.00 -> 1.86 ms; polarised 300,000: 1.89 -> 1.32).
+// * mcs_autotune times a capped copy of the cases as the part of the walk that
+//   it is: with the whole walk's chunks (tune_chunk) where that takes the queue.
 // * Walks that have a lane for every photon (replays without phase matrices,
 //   native walks) take the ONE form of k_walk: as many blocks as are resident
 //   together, the photons spread evenly over them.  Kernel ms at the default
@@ -1682,7 +1685,7 @@ static WalkShape walk_shape(const mcs_ctx *c, int mode)
         per_cu *= s.block / PolarWalker::MAX_BLOCK;   // same threads per CU in smaller blocks
         s.block = PolarWalker::MAX_BLOCK;
     }
-    if (!(replay && c->polar) && n > 0) {
+    if (!(replay && c->polar) && n > 0 && !c->tune_chunk) {
         int block = s.block, blocks = std::min(per_cu, (replay ? 4 * ReplayWalker::WAVES_PER_EU : 16) / (s.block / 64));
         if (polar) {
             const bool eight = n <= (int64_t)512 * c->cus;
@@ -1707,8 +1710,8 @@ static WalkShape walk_shape(const mcs_ctx *c, int mode)
     }
     s.take = 0;
     s.grid = per_cu * c->cus;
-    s.chunk = std::max(c->launch.chunk, c->launch.block);
-    if (replay || polar || coop == 0) {
+    s.chunk = c->tune_chunk ? c->tune_chunk : std::max(c->launch.chunk, c->launch.block);
+    if (!c->tune_chunk && (replay || polar || coop == 0)) {
         const int64_t per_block = (n + s.grid - 1) / s.grid;
         s.chunk = (int)std::min<int64_t>(s.chunk, std::max<int64_t>(per_block, c->launch.block));
     }
@@ -2269,6 +2272,17 @@ int mcs_autotune(mcs_ctx *c, const mcs_launch *cand, int32_t n, int64_t photons_
     if (photons_cap > 0)
         for (auto &k : capped) k.n_photons = std::min<int64_t>(k.n_photons, photons_cap);
     const mcs_launch keep = c->launch;
+    // candidates are for the whole walk: where it takes the chunk queue, so does
+    // the capped one, which by itself might have a lane for every photon and the
+    // same launch for every candidate
+    std::vector<int> queue_chunk((size_t)n, 0);
+    bool cut = false;
+    for (size_t k = 0; k < saved.size(); ++k) cut |= capped[k].n_photons < saved[k].n_photons;
+    for (int k = 0; cut && k < n; ++k) {
+        if (int e = mcs_set_launch(c, &cand[k])) { c->launch = keep; return e; }
+        const WalkShape whole = walk_shape(c, MCS_NATIVE);
+        queue_chunk[k] = whole.take > 0 ? 0 : whole.chunk;
+    }
     // the phase-matrix state survives the capped copy (aspherical cases are
     // timed with their own kernel)
     const std::vector<DevCase> pdc = c->dcases;
@@ -2283,6 +2297,7 @@ int mcs_autotune(mcs_ctx *c, const mcs_launch *cand, int32_t n, int64_t photons_
     int best_i = -1;
     for (int k = 0; k < n; ++k) {
         if ((r = mcs_set_launch(c, &cand[k]))) break;
+        c->tune_chunk = queue_chunk[k];
         mcs_walk_args a;
         memset(&a, 0, sizeof a);
         a.mode = MCS_NATIVE;
@@ -2301,6 +2316,7 @@ int mcs_autotune(mcs_ctx *c, const mcs_launch *cand, int32_t n, int64_t photons_
         if (times_ms) times_ms[k] = med;
         if (med < best_t) { best_t = med; best_i = k; }
     }
+    c->tune_chunk = 0;
     int r2 = mcs_set_cases(c, saved.data(), (int32_t)saved.size(), bands.data(), (int32_t)bands.size());
     if (!r2) r2 = restore_polar(c, pdc, pdb, polar, pm_n, pm_floats);
     if (r) { c->launch = keep; return r; }
