@@ -18,10 +18,11 @@ def walker():
 
 @pytest.mark.parametrize('kind', ['polar', 'reproducible'])
 def test_capped_candidates_differ(walker, tmp_path, kind):
-    """40,000 of 1e6 photons in chunks of 256 (157 blocks) and of 8,192 (5
-    blocks of 256 threads, 32 rounds of photons through each lane's queue)."""
+    """40,000 photons in chunks of 256 (157 blocks) and of 8,192 (5 blocks of 256
+    threads, 32 rounds of photons through each lane), as a walk of 8.4e6 takes them
+    (below 8,192 photons a block of the grid the larger chunks would shrink)."""
     from monte_carlompi_amd.workloads import snow_polar_case
-    n = 1_000_000
+    n = 8_192 * 4 * walker.cus
     case = snow_polar_case(n, str(tmp_path)) if kind == 'polar' else gpu_case(n, 20.0, 30.0, True, 0.5, g=0.87, ssa=0.995)
     walker.set_cases([case])
     coop = 16 if kind == 'polar' else 0
