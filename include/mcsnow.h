@@ -116,8 +116,15 @@ typedef struct {
  * sums: the same law (statistics agree), but which photons take that path
  * depends on scheduling, so records are not bit-reproducible. */
 typedef struct {
-    int32_t block;             /* threads per block: 64..1024, multiple of 64 */
-    int32_t blocks_per_cu;     /* grid = blocks_per_cu * CUs                  */
+    int32_t block;             /* threads per block: 64..1024, multiple of 64.
+                                  Polarised walks of up to 512 photons per CU
+                                  use 512, of up to 768 photons 256, whatever is
+                                  set; replays at most 256, polarised walks at
+                                  most 512                                    */
+    int32_t blocks_per_cu;     /* grid = blocks_per_cu * CUs.  Walks that are
+                                  dealt out once (below) use at most 16 waves
+                                  per CU of it (replays 8), polarised ones 1 x
+                                  512 or 3 x 256 threads                      */
     int32_t chunk;             /* photons per work-queue chunk, 64..2^24;
                                   a walk raises it to `block` when smaller.  A
                                   block keeps 4 chunks in flight and a chunk
@@ -327,7 +334,10 @@ int mcs_last_stats(const mcs_ctx *ctx, mcs_stats *out);
 
 /* Time each launch shape of `candidates` on the cases currently set (native
  * mode, records off, `photons_cap` photons per case at most, `repeats`
- * timed runs each) and keep the fastest.  times_ms (optional, n entries)
+ * timed runs each) and keep the fastest.  A capped walk takes the chunk queue
+ * where the whole one does.  Cases so small that the whole walk is dealt out once
+ * (mcs_launch.chunk) may run the same launch for several candidates: the choice
+ * among those says nothing.  times_ms (optional, n entries)
  * receives the median time of each candidate.  No reference counterpart:
  * the reference has a fixed rank count chosen by the user (README:54). */
 int mcs_autotune(mcs_ctx *ctx, const mcs_launch *candidates, int32_t n,

@@ -708,7 +708,9 @@ static void backward_pass(mcs_mlp *c, int rows, float *loss_out)
 // batch 4096 and 9 -> 4 x 256 -> 651 on MI355X k_train_rows takes 28 us,
 // k_train_dw 12 and k_train_adam 7 (the per-layer kernels, which other widths,
 // deeper or wider-output networks use: 26 launches, 234 us); 48 steps with
-// their uploads 11.2 -> 2.45 ms.
+// their uploads 11.2 -> 2.55 ms.  Layers, us a step here / there: 1 35 / 100, 2 40 /
+// 146, 3 44 / 184, 5 56 / 268, 6 67 / 310, 7 78 / 353, 8 88 / 395 (from five on the
+// pre-activations spill, 14 to 82 registers); batch 64 takes 26-65 / 62-241.
 static void pack_weights(mcs_mlp *c)
 {
     hipLaunchKernelGGL(k_pack_weights, dim3((unsigned)((c->n_pad + 255) / 256)), dim3(256), 0, c->stream, c->pm, c->p,
